@@ -289,6 +289,42 @@ template <> __device__ __forceinline__ void mfma_chunk<f16_t>(f32x16& acc, const
     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
 }
 
+// fp32 operands on the 128 x 128 tile: each fragment is split in registers into
+// three bf16 ones whose sum it is exactly (three round-to-nearest bf16 hold 24
+// bits and more): h = bf16(x), m = bf16(x - h), l = x - h - m.  The product of
+// two such fragments is l h + h l + m m + m h + h m + h h on the bf16 matrix
+// cores, summed in fp32, h h apart from the five small ones; the three terms
+// left out are below 2^-26 |x y|.  Six 32x32x16 bf16 MFMAs (192 cycles)
+// replace eight 32x32x2 fp32 ones (512 cycles).  What bounds it is the power
+// limit (the matrix pipes are 63% busy at 1.73 GHz) and the splitting's VALU
+// work, 44 operations per fragment, against 24 MFMAs per four fragments here;
+// on the 64 x 64 and 32 x 32 tiles, with one block per wave, the splitting
+// outweighs what the MFMAs save (784-256-256-10 at 64 rows 267 -> 297 us,
+// 1024-wide layers at 1024 rows 6.65 -> 6.75 ms), so those keep the fp32 MFMAs,
+// as do the 256-row tiles, which have no registers left for it.  Measured, fp32
+// MFMAs -> this: 4096^3 971 -> 718 us (192 TFLOP/s), 8192^3 7.78 -> 5.7 ms, the
+// 4 x 2048 ragged batch 109 -> 78 ms.  Error against 64 bits (2-norm, normal
+// operands): K = 64 1.4e-7 -> 5.0e-8, K = 1024 5.7e-7 -> 1.9e-7, K = 4096
+// 1.15e-6 -> 4.0e-7, K = 8192 1.6e-6 -> 5.7e-7 (one rounding of the sum per 16
+// elements of K, not one per 2).
+constexpr bool split3_tile(int bm, int bn) { return bm == 128 && bn == 128; }
+struct Split3 {
+    u32x4 h, m, l;
+};
+// One pair of elements.  Plain VALU operations (a conversion of the pair, two
+// unpackings and two exact subtractions per level): they issue beside the
+// MFMAs, where the shorter form with v_dot2_f32_bf16 holds the matrix pipe.
+__device__ __forceinline__ void split3_pair(uint32_t x0, uint32_t x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    const float f0 = __uint_as_float(x0), f1 = __uint_as_float(x1);
+    h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{f0, f1}, bf16x2));
+    const float r0 = f0 - __uint_as_float(h << 16), r1 = f1 - __uint_as_float(h & 0xFFFF0000u);
+    m = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
+    const float t0 = r0 - __uint_as_float(m << 16), t1 = r1 - __uint_as_float(m & 0xFFFF0000u);
+    l = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{t0, t1}, bf16x2));
+}
+
 // Workgroup ids are dealt round-robin over the XCDs (each with its own L2):
 // XCD x runs blocks x, x + 8, x + 16, ...
 constexpr int kXcds = 8;
@@ -386,6 +422,9 @@ template <int W> __device__ __forceinline__ u32x4 tr_fragment(const char* region
 #ifndef PCD_MID_NS
 #define PCD_MID_NS 4
 #endif
+#ifndef PCD_MID_NS32
+#define PCD_MID_NS32 5   // fp32 128 x 128: its loop keeps one stage less in flight than the ring has room for
+#endif
 #ifndef PCD_OCC_SMALL
 #define PCD_OCC_SMALL 2
 #endif
@@ -446,7 +485,7 @@ template <int BM, int BN, int OPB = 4, bool WDIR = false> struct TileCfg {
     static constexpr int NCW = NC / KW;                    // chunks of a stage one wave takes
     static constexpr int LDS_ROWS = WD ? BM : BM + BN;     // operand rows a stage holds in LDS
     static constexpr int stage_bytes = LDS_ROWS * RB;
-    static constexpr int NS_WANT = WD ? PCD_WD_NS : BIG ? PCD_BIG_NS : MID ? PCD_MID_NS : KSW ? PCD_KSW_NS : (BM + BN >= 320) ? 3 : PCD_SMALL_NS;
+    static constexpr int NS_WANT = WD ? PCD_WD_NS : BIG ? PCD_BIG_NS : MID ? (OPB == 4 ? PCD_MID_NS32 : PCD_MID_NS) : KSW ? PCD_KSW_NS : (BM + BN >= 320) ? 3 : PCD_SMALL_NS;
     static constexpr int NS = (BIG || WD) ? NS_WANT : (NS_WANT * stage_bytes <= 80 * 1024 ? NS_WANT : 80 * 1024 / stage_bytes);   // stages in the LDS ring
     static constexpr int D = NS - 1;                       // prefetch distance (stages)
     static constexpr int OCC = BIG ? 1 : KSW ? PCD_KSW_OCC : WD ? PCD_WD_OCC : PCD_OCC_SMALL;   // workgroups per CU the registers are sized for
@@ -946,6 +985,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // output blocks per wave they rotate over NSPLIT accumulator sets (summed
     // after the loop), so consecutive MFMAs never wait on each other's result.
     constexpr bool F32OP = std::is_same<OP, float>::value;
+    constexpr bool SPLIT3 = F32OP && split3_tile(BM, BN);
     constexpr int NSPLIT = (F32OP && C::FM * C::FN < 4) ? 4 / (C::FM * C::FN) : 1;
     f32x16 accs[NSPLIT][C::FM][C::FN];
 #pragma unroll
@@ -1183,6 +1223,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         }
     };
     const int c0 = wk * C::NCW;   // this wave's first chunk of a stage
+    auto sweep = [&]() PCD_INLINE {
     for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
     stage_ready(0);
     read_frags(0, c0, fa[0], fb[0]);
@@ -1217,6 +1258,137 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         if constexpr (c + 1 < NC) read_frags((nk - 1) % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
         mfmas(fa[c & 1], fb[c & 1]);
     });
+    };
+    if constexpr (SPLIT3) {
+        // Step kt (stage kt, 16 K elements of every row): the products of A's
+        // first block row, then of its second.  One set of A's pieces is enough
+        // (a fragment is split while the other one multiplies), B's alternate
+        // between two; the splitting of the fragments the next half needs goes
+        // between the MFMAs, and their LDS reads half a step ahead of it.  The
+        // five small products sum apart from h h: rounded at their own size,
+        // they cost the sum nothing, which then takes one rounding per stage.
+        static_assert(C::NCW == 2 && C::KW == 1 && C::FM == 2 && C::FN == 2, "the 128 x 128 tile's blocks and stage");
+        f32x16 small[2][2];
+        static_for<0, 4>([&](auto X) PCD_INLINE { small[decltype(X)::value / 2][decltype(X)::value % 2] = f32x16{}; });
+        u32x4 ra[2][2], rb[2][2];   // fp32 elements of the fragments to split next
+        Split3 pa[2], pb[2][2];
+        auto load_frag = [&](int kt, int row, u32x4 (&raw)[2]) PCD_INLINE {
+            const char* st = smem + (kt % C::NS) * C::stage_bytes + row * C::RB;
+            static_for<0, 2>([&](auto Cc) PCD_INLINE {
+                raw[Cc] = *(const u32x4*)(st + swz<C::RB>(row, 2 * decltype(Cc)::value + half) * 16);
+            });
+        };
+        const int arow = wm * C::WTM + lr, brow = BM + wn * C::WTN + lr;
+        auto split_half = [&](const u32x4& raw, Split3& d, auto E) PCD_INLINE {   // two pairs
+            constexpr int e = decltype(E)::value;
+            uint32_t h0, m0, l0, h1, m1, l1;
+            split3_pair(raw[0], raw[1], h0, m0, l0);
+            split3_pair(raw[2], raw[3], h1, m1, l1);
+            // not sunk to where the products read them
+            asm volatile("" : "+v"(h0), "+v"(m0), "+v"(l0), "+v"(h1), "+v"(m1), "+v"(l1));
+            d.h[2 * e] = h0; d.m[2 * e] = m0; d.l[2 * e] = l0;
+            d.h[2 * e + 1] = h1; d.m[2 * e + 1] = m1; d.l[2 * e + 1] = l1;
+        };
+        auto split_frag = [&](const u32x4 (&raw)[2], Split3& d) PCD_INLINE {
+            split_half(raw[0], d, std::integral_constant<int, 0>{});
+            split_half(raw[1], d, std::integral_constant<int, 1>{});
+        };
+        auto piece = [](const Split3& p, int w) PCD_INLINE { return w == 0 ? p.h : w == 1 ? p.m : p.l; };
+        // Product x (0..11) of block row i: term x / 2 (smallest first) of column x % 2.
+        auto product = [&](auto I, auto Q, auto X) PCD_INLINE {
+            constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+            constexpr int i = decltype(I)::value, q = decltype(Q)::value, t = decltype(X)::value / 2, j = decltype(X)::value % 2;
+            const u32x4 av = piece(pa[i], PA[t]), bv = piece(pb[q][j], PB[t]);
+            f32x16& to = t == 5 ? accs[0][i][j] : small[i][j];
+            if constexpr (TRM) mfma_chunk<bf16_t>(to, bv, av);
+            else mfma_chunk<bf16_t>(to, av, bv);
+        };
+        // Block row i's 12 products with the splitting of two fragments, a quarter of it after every third.
+        auto half_step = [&](auto I, auto Q, const u32x4 (&r0)[2], Split3& d0, const u32x4 (&r1)[2], Split3& d1) PCD_INLINE {
+            static_for<0, 4>([&](auto G) PCD_INLINE {
+                constexpr int g = decltype(G)::value;
+                static_for<3 * g, 3 * g + 3>([&](auto X) PCD_INLINE { product(I, Q, X); });
+                split_half(g < 2 ? r0[g % 2] : r1[g % 2], g < 2 ? d0 : d1, std::integral_constant<int, g % 2>{});
+                static_for<0, 3>([&](auto) PCD_INLINE {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        // Like stage_ready, with one stage less in flight: a stage's slot is
+        // refilled after the barrier that follows its last read.
+        auto ready = [&](int next) PCD_INLINE {
+            const int later = min(C::D - 2, nk - 1 - next);
+            static_for<0, C::D - 1>([&](auto Kc) PCD_INLINE {
+                constexpr int k = decltype(Kc)::value;
+                if (later == k) wait_vmcnt<k * C::QPW>();
+            });
+            __syncthreads();
+        };
+        const std::integral_constant<int, 0> I0{};
+        const std::integral_constant<int, 1> I1{};
+        auto step = [&](auto Q, int kt) PCD_INLINE {
+            constexpr int q = decltype(Q)::value;
+            load_frag(kt + 1, arow, ra[0]);
+            load_frag(kt + 1, brow + 32, rb[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            half_step(I0, Q, ra[1], pa[1], rb[0], pb[q ^ 1][0]);
+            if (kt + 2 < nk) ready(kt + 2);
+            if (kt + 1 + C::D < nk) issue_stage(kt + 1 + C::D);
+            load_frag(kt + 1, arow + 32, ra[1]);
+            load_frag(kt + 2, brow, rb[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            half_step(I1, Q, ra[0], pa[0], rb[1], pb[q ^ 1][1]);
+        };
+        // Past the last stage the reads and splits run on whatever the ring holds, unused.
+        for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
+        stage_ready(0);
+        load_frag(0, arow, ra[0]);
+        load_frag(0, arow + 32, ra[1]);
+        load_frag(0, brow, rb[0]);
+        load_frag(0, brow + 32, rb[1]);
+        split_frag(ra[0], pa[0]);
+        split_frag(rb[0], pb[0][0]);
+        split_frag(rb[1], pb[0][1]);
+        if (nk > 1) ready(1);
+        if (C::D < nk) issue_stage(C::D);
+        load_frag(1, brow, rb[0]);
+        int kt = 0;
+        for (; kt + 1 < nk; kt += 2) {
+            step(I0, kt);
+            step(I1, kt + 1);
+        }
+        if (kt < nk) step(I0, kt);
+        static_for<0, 4>([&](auto X) PCD_INLINE { accs[0][decltype(X)::value / 2][decltype(X)::value % 2] += small[decltype(X)::value / 2][decltype(X)::value % 2]; });
+        // A result that is not finite: an operand was not (its pieces mix
+        // infinities and NaNs), it rounded up to infinity as a bf16, or the sum
+        // overflowed.  The tile then takes the whole sweep again on the fp32
+        // MFMAs, which give their own infinities and NaNs.
+        bool bad = false;
+        static_for<0, C::FM>([&](auto I) PCD_INLINE {
+            static_for<0, C::FN>([&](auto J) PCD_INLINE {
+                static_for<0, 16>([&](auto R) PCD_INLINE {
+                    bad |= !(fabsf(accs[0][decltype(I)::value][decltype(J)::value][decltype(R)::value]) <= 3.402823466e38f);
+                });
+            });
+        });
+        volatile __attribute__((address_space(3))) int* flag = (volatile __attribute__((address_space(3))) int*)smem;
+        __syncthreads();   // every wave is done reading the stage ring
+        if (tid == 0) *flag = 0;
+        __syncthreads();
+        if (bad) *flag = 1;
+        __syncthreads();
+        if (*flag) {
+            __syncthreads();
+            static_for<0, C::FM>([&](auto I) PCD_INLINE {
+                static_for<0, C::FN>([&](auto J) PCD_INLINE { accs[0][decltype(I)::value][decltype(J)::value] = f32x16{}; });
+            });
+            sweep();
+        }
+    } else {
+        sweep();
+    }
     }   // LDS-operand main loop
     static_for<1, NSPLIT>([&](auto Kc) PCD_INLINE {
 #pragma unroll

@@ -479,8 +479,8 @@ long error_phase_tiles(const pcd_model* m, int batch, Tile t) {
 }
 
 // The largest tile that still gives every CU at least two workgroups per
-// phase (a phase with fewer tiles leaves SIMDs idle: 64 x 64 beats 128 x 128
-// by 8% on the 1024-wide fp32 configuration).  256 x 256 only for 16-bit
+// phase (a phase with fewer tiles leaves SIMDs idle), or, in fp32, one of
+// 128 x 128.  256 x 256 only for 16-bit
 // operands with every layer at least 1024 wide.  A settling whose error
 // phase has fewer 64 x 64 tiles than the GPU has CUs takes the K-shared
 // 32 x 32 tile: its phases are bound by one tile's K sweep, which that tile
@@ -504,7 +504,12 @@ Tile choose_tile(const pcd_model* m, int batch) {
         for (int l = 0; l < m->L; ++l) wide = wide && m->s[l] >= 1024;
         if (wide && error_phase_tiles(m, batch, Tile{256, 256}) >= want) return Tile{256, 256};
     }
-    if (error_phase_tiles(m, batch, Tile{128, 128}) >= want) return Tile{128, 128};
+    // fp32: one 128 x 128 tile per CU is enough, since that tile multiplies in
+    // split bf16 (split3_tile) at 1.4 times the fp32 MFMAs' rate: 1024-wide
+    // layers at 1024 rows (256 such tiles) 6.65 ms with 64 x 64 tiles, 6.07 with
+    // 128 x 128; 3000-1500-700-300 at 768 rows (252) 2.06 and 2.14, at 1024 (336)
+    // 2.47 and 2.21.
+    if (error_phase_tiles(m, batch, Tile{128, 128}) >= (m->dtype == PCD_F32 ? m->cus : want)) return Tile{128, 128};
     return Tile{64, 64};
 }
 
