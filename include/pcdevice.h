@@ -400,6 +400,9 @@ int pcd_pc_model_info(const pcd_model* model, int* levels, int* sizes, int max_s
  *                16-bit models (default); 0: ordinary stores; 1: non-temporal.
  *                Results are the same.
  *   nt_load      the same for the epilogues' loads of the fp32 states.
+ *   shared_rows 1: a fixed-step settling from zero states computes the layers
+ *                  the input has not reached yet once for the whole batch (their
+ *                  states are the same for every sample); 0: sample by sample.
  *   ragged_order 1: pcd_pc_relax_ragged settles the requests in decreasing
  *                step budget (rows permuted on the device and back), so rows
  *                that stop early fill whole row tiles that drop out (default);

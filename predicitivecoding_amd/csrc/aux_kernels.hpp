@@ -193,7 +193,7 @@ __global__ void exit_kernel(const float* __restrict__ part, int ldp, int nslots,
     const int r0 = row_offsets[r], r1 = row_offsets[r + 1];
     float s = 0.f;
     for (int row = r0 + threadIdx.x; row < r1; row += blockDim.x)
-        s += sum_slots(part, ldp, nslots, row);
+        s += sum_slots(part, ldp, nslots, row, nslots);
     __shared__ float red[256];
     red[threadIdx.x] = s;
     __syncthreads();
@@ -221,7 +221,7 @@ __global__ void exit_rows_kernel(const float* __restrict__ part, int ldp, int ns
                                  float* __restrict__ last_energy, int t, int rule, float thr) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < requests; r += gridDim.x * blockDim.x) {
         if (t >= done_at[r]) continue;
-        const float e = sum_slots(part, ldp, nslots, r);
+        const float e = sum_slots(part, ldp, nslots, r, nslots);
         const float prev = prev_energy[r];
         bool stop = false;
         if (rule == 1) stop = thr > 0.f && t > 0 && (prev - e < thr * fmaxf(prev, 1e-12f));
@@ -323,8 +323,15 @@ active_tiles_kernel(const int* __restrict__ row_offsets, const int* __restrict__
 __global__ void energy_rows_kernel(const float* __restrict__ part, int ldp, int nslots, float* __restrict__ out,
                                    int rows) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
-        out[r] = sum_slots(part, ldp, nslots, r);
+        out[r] = sum_slots(part, ldp, nslots, r, nslots);
     }
+}
+
+// Every row of an fp32 state [rows x ld] from one row of it (`ld` a multiple of 4).
+__global__ void broadcast_row_kernel(const f32x4* __restrict__ src, f32x4* __restrict__ dst, int ld4, int rows) {
+    const size_t n = (size_t)rows * ld4;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        dst[i] = src[i % ld4];
 }
 
 // Layer-0 rows of a classification batch: row r is sample r / classes of x0

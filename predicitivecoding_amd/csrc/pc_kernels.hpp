@@ -113,16 +113,16 @@ struct Problem {
     int tiles;            // work units: tiles_m * tiles_n * ksplit
     int ldo;              // leading dimension of every [rows x N] epilogue operand
     const float* bias;    // ERROR/FFG: b_l [N]
-    const float* mlow;    // ERROR: fp32 state M_{l-1}
+    const float* mlow;    // ERROR: fp32 state M_{l-1}; UPDATE: fp32 state M_l before the step (read at the top layer)
     float* eout;          // ERROR: X_{l-1} = M - eta (E + lambda sign M) (nullable: layer 0 is never updated)
     void* dout;           // ERROR: D_l in the operand type; FFG: operand-type state copy
-    float* m;             // UPDATE: fp32 state M_l (in/out); FFG: state out; PLAIN: C
+    float* m;             // UPDATE: fp32 state M_l out; FFG: state out; PLAIN: C
     void* mop;            // UPDATE: operand-type copy of M_l (nullable for fp32)
     const float* eself;   // UPDATE: X_l from the error phase (nullable for the top layer)
     float prec;           // ERROR: P_{l-1}
     int slot_base;        // ERROR: first energy partial slot of this problem
     int ksplit;           // K ranges per tile (<= 1: none); the last range to finish runs the epilogue
-    int ksplit_pad;
+    int ldi;              // ERROR/UPDATE: row pitch of mlow and eself: ldo, or 0 where every row reads the first
     float* part;          // split-K: fp32 partial tiles [tiles_m * tiles_n * ksplit x BM * BN]
     int* count;           // split-K: finished ranges per tile [tiles_m * tiles_n], zero between launches
 };
@@ -158,6 +158,7 @@ struct PhaseArgs {
     int ldp, nslots;
     float* energy_out;          // UPDATE prologue: row energies of step t (nullable)
     int batch, t;
+    int shared_from;            // energy slots from this one on hold one row's energies, the same for every row
     const int* row_req;         // ragged: request of each row (nullable)
     const int* done_at;         // ragged: first step a request no longer runs
     int tile_order;             // TILE_INTERLEAVED or TILE_CONTIGUOUS (see phase_grid)
@@ -336,20 +337,25 @@ __host__ __device__ __forceinline__ void xcd_share(int n, int x, int& lo, int& c
     cnt = n * (x + 1) / kXcds - lo;
 }
 
-// Sum of a row's energy partials over the slots, in slot order.  The loads
-// go out eight at a time ahead of the adds (one dependent load per slot would
-// pay the memory latency nslots times).
-__device__ __forceinline__ float sum_slots(const float* part, int ldp, int nslots, int row) {
+// Sum of a row's energy partials over the slots, in slot order (slots from
+// shared_from on are row 0's for every row).  The loads go out eight at a time
+// ahead of the adds (one dependent load per slot would pay the memory latency
+// nslots times).
+__device__ __forceinline__ float sum_slots(const float* part, int ldp, int nslots, int row, int shared_from) {
     float s = 0.f;
     int k = 0;
-    for (; k + 8 <= nslots; k += 8) {
-        float v[8];
+    auto add = [&](const float* at, int end) PCD_INLINE {
+        for (; k + 8 <= end; k += 8) {
+            float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = gld(part + (size_t)(k + j) * ldp + row);
+            for (int j = 0; j < 8; ++j) v[j] = gld(at + (size_t)(k + j) * ldp);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s += v[j];
-    }
-    for (; k < nslots; ++k) s += gld(part + (size_t)k * ldp + row);
+            for (int j = 0; j < 8; ++j) s += v[j];
+        }
+        for (; k < end; ++k) s += gld(at + (size_t)k * ldp);
+    };
+    add(part + row, shared_from);
+    if (shared_from < nslots) add(part, nslots);
     return s;
 }
 
@@ -883,7 +889,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     if (EPI == EPI_UPDATE && args.energy_out != nullptr) {
         for (int row = (vgrid - 1 - vblock) * C::NT + tid; row < args.batch; row += vgrid * C::NT) {
             gst(args.energy_out + (size_t)args.t * args.batch + row,
-                sum_slots(args.energy_part, args.ldp, args.nslots, row));
+                sum_slots(args.energy_part, args.ldp, args.nslots, row, args.shared_from));
         }
     }
 
@@ -971,12 +977,12 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // latency passes under the K sweep.
     f32x4 epi_state{}, epi_bias{};
     if constexpr (C::KW > 1 && (EPI == EPI_ERROR || EPI == EPI_UPDATE)) {
-        const size_t eidx = (size_t)(row0 + (lane & 31)) * P.ldo + col0 + 8 * wave + 4 * (lane >> 5);
+        const size_t eidx = (size_t)(row0 + (lane & 31)) * P.ldi + col0 + 8 * wave + 4 * (lane >> 5);
         if constexpr (EPI == EPI_ERROR) {
             epi_state = gld4(P.mlow + eidx);
             epi_bias = gld4(P.bias + col0 + 8 * wave + 4 * (lane >> 5));
         } else {
-            epi_state = gld4((P.eself != nullptr ? P.eself : P.m) + eidx);
+            epi_state = gld4((P.eself != nullptr ? P.eself : P.mlow) + eidx);
         }
     }
 
@@ -1223,42 +1229,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         }
     };
     const int c0 = wk * C::NCW;   // this wave's first chunk of a stage
-    auto sweep = [&]() PCD_INLINE {
-    for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
-    stage_ready(0);
-    read_frags(0, c0, fa[0], fb[0]);
-    // Chunk c's MFMAs run while chunk c+1's fragments are read; the last chunk
-    // of a stage runs after the barrier that publishes the next stage, whose
-    // first fragments it overlaps.  The last stage is peeled off.
-    for (int kt = 0; kt + 1 < nk; ++kt) {
-        if (kt + C::D < nk) issue_stage(kt + C::D);
-        if constexpr (NC == 1) {
-            // One chunk per wave and stage (the K-shared tile on 16-bit
-            // operands): its MFMA runs across the barrier, and the next
-            // stage's fragments are read into the same registers after it.
-            mfmas(fa[0], fb[0]);
-            stage_ready(kt + 1);
-            read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
-        } else {
-            static_for<0, NC>([&](auto Cc) PCD_INLINE {
-                constexpr int c = decltype(Cc)::value;
-                if constexpr (c + 1 < NC) {
-                    read_frags(kt % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
-                } else {
-                    stage_ready(kt + 1);
-                    read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
-                }
-                mfmas(fa[c & 1], fb[c & 1]);
-                interleave();
-            });
-        }
-    }
-    static_for<0, NC>([&](auto Cc) PCD_INLINE {
-        constexpr int c = decltype(Cc)::value;
-        if constexpr (c + 1 < NC) read_frags((nk - 1) % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
-        mfmas(fa[c & 1], fb[c & 1]);
-    });
-    };
+    bool op_mfmas = true;   // the sweep on the operand type's own MFMAs
     if constexpr (SPLIT3) {
         // Step kt (stage kt, 16 K elements of every row): the products of A's
         // first block row, then of its second.  One set of A's pieces is enough
@@ -1365,11 +1336,15 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         // infinities and NaNs), it rounded up to infinity as a bf16, or the sum
         // overflowed.  The tile then takes the whole sweep again on the fp32
         // MFMAs, which give their own infinities and NaNs.
+        // (A settling's rows past M hold what earlier calls left there and do not
+        // count.)
         bool bad = false;
         static_for<0, C::FM>([&](auto I) PCD_INLINE {
             static_for<0, C::FN>([&](auto J) PCD_INLINE {
                 static_for<0, 16>([&](auto R) PCD_INLINE {
-                    bad |= !(fabsf(accs[0][decltype(I)::value][decltype(J)::value][decltype(R)::value]) <= 3.402823466e38f);
+                    constexpr int i = decltype(I)::value, j = decltype(J)::value, r = decltype(R)::value;
+                    bad |= (!TRM || row0 + wm * C::WTM + i * 32 + lr < P.M) &&
+                           !(fabsf(accs[0][i][j][r]) <= 3.402823466e38f);
                 });
             });
         });
@@ -1379,15 +1354,49 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         __syncthreads();
         if (bad) *flag = 1;
         __syncthreads();
-        if (*flag) {
+        op_mfmas = *flag != 0;
+        if (op_mfmas) {
             __syncthreads();
             static_for<0, C::FM>([&](auto I) PCD_INLINE {
                 static_for<0, C::FN>([&](auto J) PCD_INLINE { accs[0][decltype(I)::value][decltype(J)::value] = f32x16{}; });
             });
-            sweep();
         }
-    } else {
-        sweep();
+    }
+    if (op_mfmas) {
+    for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
+    stage_ready(0);
+    read_frags(0, c0, fa[0], fb[0]);
+    // Chunk c's MFMAs run while chunk c+1's fragments are read; the last chunk
+    // of a stage runs after the barrier that publishes the next stage, whose
+    // first fragments it overlaps.  The last stage is peeled off.
+    for (int kt = 0; kt + 1 < nk; ++kt) {
+        if (kt + C::D < nk) issue_stage(kt + C::D);
+        if constexpr (NC == 1) {
+            // One chunk per wave and stage (the K-shared tile on 16-bit
+            // operands): its MFMA runs across the barrier, and the next
+            // stage's fragments are read into the same registers after it.
+            mfmas(fa[0], fb[0]);
+            stage_ready(kt + 1);
+            read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
+        } else {
+            static_for<0, NC>([&](auto Cc) PCD_INLINE {
+                constexpr int c = decltype(Cc)::value;
+                if constexpr (c + 1 < NC) {
+                    read_frags(kt % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
+                } else {
+                    stage_ready(kt + 1);
+                    read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
+                }
+                mfmas(fa[c & 1], fb[c & 1]);
+                interleave();
+            });
+        }
+    }
+    static_for<0, NC>([&](auto Cc) PCD_INLINE {
+        constexpr int c = decltype(Cc)::value;
+        if constexpr (c + 1 < NC) read_frags((nk - 1) % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
+        mfmas(fa[c & 1], fb[c & 1]);
+    });
     }
     }   // LDS-operand main loop
     static_for<1, NSPLIT>([&](auto Kc) PCD_INLINE {
@@ -1573,7 +1582,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
             f32x4 mraw[PD][4];
             auto load_block = [&](auto Bc) PCD_INLINE {
                 constexpr int b = decltype(Bc)::value, i = b / C::FN, j = b % C::FN;
-                load_block_rows<GNT>(mraw[b % PD], P.mlow, ldo, row0 + wm * C::WTM + i * 32, col0 + wn * C::WTN + j * 32,
+                load_block_rows<GNT>(mraw[b % PD], P.mlow, P.ldi, row0 + wm * C::WTM + i * 32, col0 + wn * C::WTN + j * 32,
                                 P.M, P.N, ntld);
             };
             static_for<0, PD>([&](auto Bc) PCD_INLINE { load_block(Bc); });
@@ -1685,14 +1694,14 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         constexpr int NB = C::FM * C::FN, PD = NB < 3 ? NB : 3;
         const float eta = args.eta, lam = args.act_reg;
         const bool folded = P.eself != nullptr;
-        const float* src = folded ? P.eself : P.m;
+        const float* src = folded ? P.eself : P.mlow;
         auto update = [&](auto FullC, auto GntC) PCD_INLINE {
         constexpr bool FULL = decltype(FullC)::value;
         constexpr bool GNT = decltype(GntC)::value;   // non-temporal global loads and stores
         f32x4 xraw[PD][4];
         auto load_block = [&](auto Bc) PCD_INLINE {
             constexpr int b = decltype(Bc)::value, i = b / C::FN, j = b % C::FN;
-            load_block_rows<GNT>(xraw[b % PD], src, ldo, row0 + wm * C::WTM + i * 32, col0 + wn * C::WTN + j * 32,
+            load_block_rows<GNT>(xraw[b % PD], src, P.ldi, row0 + wm * C::WTM + i * 32, col0 + wn * C::WTN + j * 32,
                                  P.M, P.N, ntld, FULL);
         };
         static_for<0, PD>([&](auto Bc) PCD_INLINE { load_block(Bc); });
