@@ -40,11 +40,16 @@ __global__ void zero_segs_kernel(const ZeroSegs z) {
 // bit.  A workgroup moves 64 x 64 tiles through LDS, so the source reads and
 // the destination writes are both row-contiguous whichever way the source is
 // read (one element per thread straight across a transpose reads one element
-// per 2-byte segment of a row).
+// per 2-byte segment of a row).  `items` such matrices lie back to back, source
+// and destination (prow * ldd elements apart) alike.
 template <typename OP>
-__global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ src, int src_is_f32, int rows, int cols,
-                                                   int trans, void* __restrict__ dst, int prow, int pcol, int ldd) {
+__global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ src0, int src_is_f32, int rows, int cols,
+                                                   int trans, void* __restrict__ dst0, int prow, int pcol, int ldd,
+                                                   int items) {
     __shared__ uint32_t tile[64][65];   // raw bits: fp32 values or 16-bit codes; 65 words a row, conflict-free
+    for (int item = blockIdx.z; item < items; item += gridDim.z) {
+    const void* src = (const char*)src0 + (size_t)item * rows * cols * (src_is_f32 ? 4 : 2);
+    void* dst = (char*)dst0 + (size_t)item * prow * ldd * OpTraits<OP>::bytes;
     // Thread t moves 4 consecutive elements of a row: row t/16 (+16, +32, +48), elements 4 (t%16) .. +3.
     const int q4 = (threadIdx.x & 15) * 4, qr = threadIdx.x >> 4;
     const int c0 = blockIdx.x * 64, tiles_y = (prow + 63) / 64;
@@ -108,6 +113,7 @@ __global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ src,
         }
         __syncthreads();   // the next tile row reuses `tile`
     }
+    }
 }
 
 // Fragment-major copy of a 16-bit operand [rows x cols] with rows `ld`
@@ -125,28 +131,6 @@ __global__ void frag_pack_kernel(const u32x4* __restrict__ src, int ld, int rows
         const int kc = (int)(f % kcs), rb = (int)(f / kcs);
         const int r = rb * 32 + lane % 32;
         dst[i] = src[((size_t)r * ld + (size_t)kc * 16 + 8 * (lane / 32)) / 8];
-    }
-}
-
-// pack_kernel over `batch` matrices stored back to back: item i of src is the
-// [rows x cols] matrix (or [cols x rows] read transposed) at src + i * rows *
-// cols, packed into the zero-padded [prow x pcol] buffer at dst + i * prow *
-// pcol (row pitch pcol).
-template <typename OP>
-__global__ void pack_batched_kernel(const void* __restrict__ src, int src_is_f32, int batch, int rows, int cols,
-                                    int trans, void* __restrict__ dst, int prow, int pcol) {
-    const size_t per = (size_t)prow * pcol, n = per * batch, src_per = (size_t)rows * cols;
-    for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x) {
-        const size_t item = k / per, e = k % per;
-        const int r = (int)(e / pcol), c = (int)(e % pcol);
-        const bool inside = r < rows && c < cols;
-        const size_t s = item * src_per + (trans ? (size_t)c * rows + r : (size_t)r * cols + c);
-        if (src_is_f32) {
-            OpTraits<OP>::store(dst, k, inside ? ((const float*)src)[s] : 0.f);
-        } else {
-            // 16-bit source of the operand's own type: copy the bits
-            ((uint16_t*)dst)[k] = inside ? ((const uint16_t*)src)[s] : (uint16_t)0;
-        }
     }
 }
 

@@ -73,8 +73,9 @@ enum Act { ACT_LINEAR = 0, ACT_TANH = 1, ACT_RELU = 2, ACT_SIGMOID = 3, ACT_GELU
 // layout of Gemm.MatMul's B), read where it lies: each stage's K rows of the
 // tile's columns go into LDS as they are and the MFMA fragments come out of
 // them through gfx950's transposing LDS read (ds_read_b64_tr_b16), so the
-// operand is never packed.  EPI_PLAIN_MK: the same for an A stored [K x M]
-// (a transposed A); EPI_PLAIN_MKKN: both.  16-bit operands, LDS-operand tiles.
+// operand is never packed (fp32 fragments are read an element at a time, 32
+// columns in a row).  EPI_PLAIN_MK: the same for an A stored [K x M]
+// (a transposed A); EPI_PLAIN_MKKN: both.  LDS-operand tiles.
 enum Epi { EPI_ERROR = 0, EPI_UPDATE = 1, EPI_FFG = 2, EPI_PLAIN = 3, EPI_PLAIN_KN = 4, EPI_PLAIN_MK = 5,
            EPI_PLAIN_MKKN = 6 };
 
@@ -154,6 +155,8 @@ struct PhaseArgs {
     int act;
     float eta, act_reg;
     float alpha, beta;          // PLAIN
+    int items, item_tiles;      // PLAIN: products of the launch's one shape (<= 1: one) and the work units of each
+    size_t item_a, item_b, item_c;   // PLAIN: bytes from one product's A, B to the next, elements of its C
     float* energy_part;         // [nslots x ldp] per-row partial energies (nullable)
     int ldp, nslots;
     float* energy_out;          // UPDATE prologue: row energies of step t (nullable)
@@ -384,6 +387,31 @@ template <int RB> __device__ __forceinline__ int swz(int row, int unit) {
 // halves, and the XOR separates k and k + 2.
 template <int BN> __device__ __forceinline__ int kn_swz(int k) {
     return BN >= 128 ? (k & 3) * 4 : ((k >> 1) & 1) * 4;
+}
+// Where the K rows of W elements of such a stage region lie: logical K row of
+// a physical row (and back: both maps are their own inverse), and logical
+// 16-byte unit of a physical one in it.  fp32: a fragment read takes 32
+// consecutive columns of K rows k (lanes 0-31) and k + 4 (lanes 32-63) in one
+// access, so those two rows go on different halves of the 64 banks, by the
+// unit where a row fills a bank period, by the row's place where it is half one.
+template <int W, int OPB> __device__ __forceinline__ int kn_row(int k) {
+    return OPB == 4 && W == 32 ? k ^ ((k >> 2) & 1) : k;
+}
+template <int W, int OPB> __device__ __forceinline__ int kn_unit(int k, int unit) {
+    if constexpr (OPB == 2) return unit ^ kn_swz<W>(k);
+    else return W == 32 ? unit : unit ^ (((k >> 2) & 1) * 8);
+}
+// This lane's four fp32 elements of chunk c (K rows 8c + 4 (lane / 32) ..+3)
+// at column x0 + lane % 32, from a region of K rows of W elements.
+template <int W> __device__ __forceinline__ u32x4 col_fragment(const char* region, int c, int x0) {
+    const int lane = threadIdx.x & 63, x = x0 + (lane & 31);
+    u32x4 v;
+    static_for<0, 4>([&](auto E) PCD_INLINE {
+        const int k = 8 * c + 4 * (lane >> 5) + decltype(E)::value;
+        const char* p = region + kn_row<W, 4>(k) * (W * 4) + kn_unit<W, 4>(k, x >> 2) * 16 + (x & 3) * 4;
+        v[decltype(E)::value] = *(const uint32_t*)p;
+    });
+    return v;
 }
 // One 32 x 32 x 16 MFMA operand fragment from a stage region that holds K
 // rows of W 16-bit elements (a row-major B, or a transposed A), laid out by
@@ -937,7 +965,16 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         }
     }
     if (local < 0) return;  // a spare workgroup of this XCD (the grid is 8 x the largest XCD share)
-    const Problem P = load_problem(kprobs + p);
+    Problem P = load_problem(kprobs + p);
+    if constexpr (EPI >= EPI_PLAIN) {
+        if (args.items > 1) {   // one of several products of the same shape
+            const int item = local / args.item_tiles;
+            local -= item * args.item_tiles;
+            P.A = (const char*)P.A + item * args.item_a;
+            P.B = (const char*)P.B + item * args.item_b;
+            P.m += item * args.item_c;
+        }
+    }
     // Split-K: unit `local` is K range `split` of tile `local / ksplit` (a
     // tile's ranges are consecutive units: mostly on one XCD, but an XCD's
     // share may end inside a tile, so the handshake below does not rely on it).
@@ -1017,8 +1054,8 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // row.  A stored [K x M] (EPI_PLAIN_MK, _MKKN) likewise, with lda and row0.
     constexpr bool BKN = EPI == EPI_PLAIN_KN || EPI == EPI_PLAIN_MKKN;
     constexpr bool AKM = EPI == EPI_PLAIN_MK || EPI == EPI_PLAIN_MKKN;
-    static_assert(!(AKM || BKN) || (OPB == 2 && C::KW == 1 && !C::WD),
-                  "operands read through transposing LDS reads: 16-bit operands, LDS-operand tiles");
+    static_assert(!(AKM || BKN) || (!C::WD && (OPB == 4 || C::KW == 1)),
+                  "operands in K rows: LDS-operand tiles, the K-shared one in fp32 only");
     const size_t lda_b = (size_t)P.lda * OPB, ldb_b = (size_t)P.ldb * OPB;
     const char* Ag = AKM ? (const char*)P.A + (size_t)row0 * OPB + (size_t)kb * KE * lda_b
                          : (const char*)P.A + (size_t)row0 * lda_b + (size_t)kb * C::RB;
@@ -1123,14 +1160,23 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         const int q = wave_u * C::QPW + i;
         const int R = q * C::ROWS_PER_LOAD + lane / C::UNITS;
         const int unit = swz<C::RB>(R, lane % C::UNITS);
+        // A product's last tiles repeat its last row, or the last unit of a K
+        // row, where they reach past it (those results are not stored), so the
+        // caller's operands need no whole tiles.
+        constexpr int UE = 16 / OPB;   // elements of a unit
         if (BKN && R >= BM) {
             const int ob = (q * C::ROWS_PER_LOAD - BM) * C::RB + lane * 16;
-            const int kr = ob / (BN * OPB);
-            src[i] = Bg + (size_t)kr * ldb_b + ((ob % (BN * OPB)) / 16 ^ kn_swz<BN>(kr)) * 16;
+            const int kr = kn_row<BN, OPB>(ob / (BN * OPB));
+            const int at = kn_unit<BN, OPB>(kr, (ob % (BN * OPB)) / 16) * UE;
+            src[i] = Bg + (size_t)kr * ldb_b + (ptrdiff_t)(min(col0 + at, P.N - UE) - col0) * OPB;
         } else if (AKM && R < BM) {
             const int ob = q * C::ROWS_PER_LOAD * C::RB + lane * 16;
-            const int kr = ob / (BM * OPB);
-            src[i] = Ag + (size_t)kr * lda_b + ((ob % (BM * OPB)) / 16 ^ kn_swz<BM>(kr)) * 16;
+            const int kr = kn_row<BM, OPB>(ob / (BM * OPB));
+            const int at = kn_unit<BM, OPB>(kr, (ob % (BM * OPB)) / 16) * UE;
+            src[i] = Ag + (size_t)kr * lda_b + (ptrdiff_t)(min(row0 + at, P.M - UE) - row0) * OPB;
+        } else if (EPI >= EPI_PLAIN) {
+            src[i] = (R < BM ? Ag + (size_t)(min(row0 + R, P.M - 1) - row0) * lda_b
+                             : Bg + (size_t)(min(col0 + R - BM, P.N - 1) - col0) * ldb_b) + unit * 16;
         } else {
             src[i] = R < BM ? Ag + (size_t)R * lda_b + unit * 16 : Bg + (size_t)(R - BM) * ldb_b + unit * 16;
         }
@@ -1152,7 +1198,9 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         const char* st = smem + slot * C::stage_bytes;
 #pragma unroll
         for (int i = 0; i < C::FM; ++i) {
-            if constexpr (AKM) {
+            if constexpr (AKM && F32OP) {
+                a[i] = col_fragment<BM>(st, c, wm * C::WTM + i * 32);
+            } else if constexpr (AKM) {
                 a[i] = tr_fragment<BM>(st, c, wm * C::WTM + i * 32);
             } else {
                 const int R = wm * C::WTM + i * 32 + lr;
@@ -1161,7 +1209,9 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         }
 #pragma unroll
         for (int j = 0; j < C::FN; ++j) {
-            if constexpr (BKN) {
+            if constexpr (BKN && F32OP) {
+                b[j] = col_fragment<BN>(st + BM * C::RB, c, wn * C::WTN + j * 32);
+            } else if constexpr (BKN) {
                 b[j] = tr_fragment<BN>(st + BM * C::RB, c, wn * C::WTN + j * 32);
             } else {
                 const int R = BM + wn * C::WTN + j * 32 + lr;
@@ -1208,7 +1258,8 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // One LDS fragment read after each of the chunk's first MFMAs, the rest of
     // the MFMAs after them.
     constexpr int NMF = C::FM * C::FN * (F32OP ? 4 : 1);   // MFMAs per chunk
-    constexpr int NRD = C::FM * (AKM ? 2 : 1) + C::FN * (BKN ? 2 : 1);   // fragment reads per chunk
+    constexpr int KRD = F32OP ? 4 : 2;   // reads per fragment of an operand in K rows
+    constexpr int NRD = C::FM * (AKM ? KRD : 1) + C::FN * (BKN ? KRD : 1);   // fragment reads per chunk
     auto interleave = [&]() PCD_INLINE {
         // MFMA first: the chunk's first MFMA then waits only on fragments read
         // before it, not on the read just issued (bf16 phases +1%).
@@ -1243,13 +1294,25 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         static_for<0, 4>([&](auto X) PCD_INLINE { small[decltype(X)::value / 2][decltype(X)::value % 2] = f32x16{}; });
         u32x4 ra[2][2], rb[2][2];   // fp32 elements of the fragments to split next
         Split3 pa[2], pb[2][2];
-        auto load_frag = [&](int kt, int row, u32x4 (&raw)[2]) PCD_INLINE {
-            const char* st = smem + (kt % C::NS) * C::stage_bytes + row * C::RB;
+        // Block row i of this wave's part of A, or block column i of B.
+        auto load_a = [&](int kt, int i, u32x4 (&raw)[2]) PCD_INLINE {
+            const char* st = smem + (kt % C::NS) * C::stage_bytes;
+            const int row = wm * C::WTM + i * 32 + lr;
             static_for<0, 2>([&](auto Cc) PCD_INLINE {
-                raw[Cc] = *(const u32x4*)(st + swz<C::RB>(row, 2 * decltype(Cc)::value + half) * 16);
+                constexpr int c = decltype(Cc)::value;
+                if constexpr (AKM) raw[c] = col_fragment<BM>(st, c, wm * C::WTM + i * 32);
+                else raw[c] = *(const u32x4*)(st + row * C::RB + swz<C::RB>(row, 2 * c + half) * 16);
             });
         };
-        const int arow = wm * C::WTM + lr, brow = BM + wn * C::WTN + lr;
+        auto load_b = [&](int kt, int j, u32x4 (&raw)[2]) PCD_INLINE {
+            const char* st = smem + (kt % C::NS) * C::stage_bytes;
+            const int row = BM + wn * C::WTN + j * 32 + lr;
+            static_for<0, 2>([&](auto Cc) PCD_INLINE {
+                constexpr int c = decltype(Cc)::value;
+                if constexpr (BKN) raw[c] = col_fragment<BN>(st + BM * C::RB, c, wn * C::WTN + j * 32);
+                else raw[c] = *(const u32x4*)(st + row * C::RB + swz<C::RB>(row, 2 * c + half) * 16);
+            });
+        };
         auto split_half = [&](const u32x4& raw, Split3& d, auto E) PCD_INLINE {   // two pairs
             constexpr int e = decltype(E)::value;
             uint32_t h0, m0, l0, h1, m1, l1;
@@ -1301,30 +1364,30 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         const std::integral_constant<int, 1> I1{};
         auto step = [&](auto Q, int kt) PCD_INLINE {
             constexpr int q = decltype(Q)::value;
-            load_frag(kt + 1, arow, ra[0]);
-            load_frag(kt + 1, brow + 32, rb[1]);
+            load_a(kt + 1, 0, ra[0]);
+            load_b(kt + 1, 1, rb[1]);
             __builtin_amdgcn_sched_barrier(0);
             half_step(I0, Q, ra[1], pa[1], rb[0], pb[q ^ 1][0]);
             if (kt + 2 < nk) ready(kt + 2);
             if (kt + 1 + C::D < nk) issue_stage(kt + 1 + C::D);
-            load_frag(kt + 1, arow + 32, ra[1]);
-            load_frag(kt + 2, brow, rb[0]);
+            load_a(kt + 1, 1, ra[1]);
+            load_b(kt + 2, 0, rb[0]);
             __builtin_amdgcn_sched_barrier(0);
             half_step(I1, Q, ra[0], pa[0], rb[1], pb[q ^ 1][1]);
         };
         // Past the last stage the reads and splits run on whatever the ring holds, unused.
         for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
         stage_ready(0);
-        load_frag(0, arow, ra[0]);
-        load_frag(0, arow + 32, ra[1]);
-        load_frag(0, brow, rb[0]);
-        load_frag(0, brow + 32, rb[1]);
+        load_a(0, 0, ra[0]);
+        load_a(0, 1, ra[1]);
+        load_b(0, 0, rb[0]);
+        load_b(0, 1, rb[1]);
         split_frag(ra[0], pa[0]);
         split_frag(rb[0], pb[0][0]);
         split_frag(rb[1], pb[0][1]);
         if (nk > 1) ready(1);
         if (C::D < nk) issue_stage(C::D);
-        load_frag(1, brow, rb[0]);
+        load_b(1, 0, rb[0]);
         int kt = 0;
         for (; kt + 1 < nk; kt += 2) {
             step(I0, kt);

@@ -559,12 +559,13 @@ int max_energy_slots(const pcd_model* m) {
 // walks down several tile rows when the matrix is large).
 template <typename OP>
 void pack_op(hipStream_t s, const void* src, int src_is_f32, int rows, int cols, int trans, void* dst, int prow,
-             int pcol, int ldd) {
+             int pcol, int ldd, int items = 1) {
     const int tiles_x = (pcol + 63) / 64, tiles_y = (prow + 63) / 64;
     const int gy = std::max(1, std::min({tiles_y, 65535, (4096 + tiles_x - 1) / tiles_x}));
-    const dim3 grid((unsigned)tiles_x, (unsigned)gy);
+    const int gz = std::max(1, std::min({items, 65535, 4096 / std::max(1, tiles_x * gy)}));
+    const dim3 grid((unsigned)tiles_x, (unsigned)gy, (unsigned)gz);
     hipLaunchKernelGGL(pack_kernel<OP>, grid, dim3(256), 0, s, src, src_is_f32, rows, cols, trans, dst, prow, pcol,
-                       ldd);
+                       ldd, items);
 }
 
 // Split-K.  A phase whose output tiles leave CUs idle (at most half as many
@@ -1534,182 +1535,123 @@ static Tile choose_gemm_tile(int dtype, int m, int n, int cus, int batch = 1) {
     return Tile{64, 64};
 }
 
-static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int m, int k, int n, int trans_a,
-                       int trans_b, float beta, void* stream_) {
+// `batch` products C_i = op(A_i) op(B_i) + beta C_i of one shape, items m k, k n
+// and m n elements apart, row-major.
+//
+// An operand is read where it lies when the kernel can: K a whole number of
+// the tile's stages and 16-byte aligned rows.  op(A) and op(B)^T K-contiguous
+// (A as given, B given transposed) go through the plain epilogue; B in
+// Gemm.MatMul's own row-major [k x n] layout and a transposed A ([k x m]) through
+// EPI_PLAIN_KN, _MK and _MKKN, which take K rows of the tile's columns.  Rows
+// and columns need no whole tiles (the kernel repeats the last ones).  Any
+// other operand is packed K-contiguous, K padded with zeros, into scratch.
+// All products run in one launch (their tiles dealt over the XCDs together).
+// Measured, packing whatever filled no whole tiles -> in place: 1000 x 1024 x
+// 4096 fp32 row-major 69 -> 62 us; 1000 x 4096 x 4096 bf16 57 -> 50 us; 96 x
+// (200 x 64 x 200) fp32, before also in six launches of 16 products, 114 -> 17 us.
+static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int batch, int m, int k, int n,
+                       int trans_a, int trans_b, float beta, void* stream_) {
     if (!dA || !dB || !dC) return fail(PCD_INVALID_VALUE, "pcd_gemm: null pointer");
-    if (m < 1 || k < 1 || n < 1) return fail(PCD_INVALID_VALUE, "pcd_gemm: bad shape %d x %d x %d", m, k, n);
-    hipStream_t s = (hipStream_t)stream_;
-    int dev = 0, cus = 256;
-    HIP_TRY(hipGetDevice(&dev));
-    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const Tile tile = choose_gemm_tile(dtype, m, n, cus);
-    const int mp = (int)round_up(m, tile.m), np = (int)round_up(n, tile.n), kp = (int)round_up(k, kFeatPad);
-    const int ob = op_bytes(dtype);
-    // An operand already K-contiguous, with whole tiles of rows, K a whole
-    // number of stages and 16-byte aligned rows, is read where it lies; any
-    // other is packed into zero-padded scratch.
-    auto aligned = [&](const void* p) { return ((uintptr_t)p % 16) == 0; };
-    const bool direct_a = !trans_a && m == mp && k == kp && aligned(dA);
-    const bool direct_b = trans_b && n == np && k == kp && aligned(dB);
-    // B in Gemm.MatMul's own row-major [k x n] layout, with whole tiles of
-    // columns and K a whole number of stages, is read where it lies too, on the
-    // 16-bit tiles that transpose it in LDS (EPI_PLAIN_KN).
-    // So is a transposed A (physical [k x m]) on those tiles (EPI_PLAIN_MK).
-    // Except that the transposing reads cost the 128 x 128 tile about a fifth
-    // of its time, more than packing an operand a quarter the other's size or
-    // smaller takes (512 x 8192 x 8192 bf16, A transposed: 0.089 ms in place,
-    // 0.081 packed; the other tiles lose 2-5% and read in place).
-    const bool small_a = tile.m == 128 && (size_t)m * 4 <= (size_t)n;
-    const bool small_b = tile.m == 128 && (size_t)n * 4 <= (size_t)m;
-    const bool kn_b = !trans_b && !small_b && kn_tile(ob, tile.m, tile.n, false) && n == np && k == kp && aligned(dB);
-    const bool mk_a = trans_a && !small_a && kn_tile(ob, tile.m, tile.n, false) && m == mp && k == kp && aligned(dA);
-    void *pa = nullptr, *pb = nullptr;
-    int st = PCD_SUCCESS;
-    auto release = [&]() {
-        if (pa && !direct_a && !mk_a) pool_free(pa, s);
-        if (pb && !direct_b && !kn_b) pool_free(pb, s);
-    };
-    const int src_f32 = dtype == PCD_F32;
-    auto pack = [&](const void* src, int rows, int cols, int trans, void* dst, int prow, int pcol) -> int {
-        switch (dtype) {
-        case PCD_F32: pack_op<float>(s, src, src_f32, rows, cols, trans, dst, prow, pcol, pcol); break;
-        case PCD_BF16: pack_op<bf16_t>(s, src, src_f32, rows, cols, trans, dst, prow, pcol, pcol); break;
-        default: pack_op<f16_t>(s, src, src_f32, rows, cols, trans, dst, prow, pcol, pcol); break;
-        }
-        return from_hip(hipGetLastError(), "pack_kernel launch");
-    };
-    // op(A) [m x k]: physical [m x k], or [k x m] when transposed.
-    // The kernel's B operand is op(B)^T [n x k]: physical B is [k x n] (read
-    // transposed) or, with trans_b, already [n x k].
-    if (direct_a || mk_a) pa = (void*)dA;
-    else if (!(st = pool_alloc(&pa, (size_t)mp * kp * ob, s))) st = pack(dA, m, k, trans_a, pa, mp, kp);
-    if (!st) {
-        if (direct_b || kn_b) pb = (void*)dB;
-        else if (!(st = pool_alloc(&pb, (size_t)np * kp * ob, s))) st = pack(dB, n, k, trans_b ? 0 : 1, pb, np, kp);
-    }
-    std::vector<ProblemSet> sets(1);
-    std::memset(&sets[0], 0, sizeof(ProblemSet));
-    sets[0].n = 1;
-    Problem& p = sets[0].p[0];
-    p.A = pa;
-    p.lda = mk_a ? m : kp;   // the row pitch of a transposed A, else of the K-contiguous rows
-    p.B = pb;
-    p.ldb = kn_b ? n : kp;   // the row pitch of row-major B, else of the K-contiguous copy
-    p.M = m;
-    p.N = n;
-    p.K = kp;
-    p.tiles_m = mp / tile.m;
-    p.tiles_n = np / tile.n;
-    p.tiles = p.tiles_m * p.tiles_n;
-    p.ldo = n;
-    p.m = dC;
-    // Split-K scratch from the pool; the counters start at zero (a fill
-    // kernel, so a captured call stays free of memset nodes).
-    SplitScratch sc;
-    void* part = nullptr;
-    if (!st && tile.m * tile.n <= 128 * 128 && p.tiles * 2 <= cus) {
-        sc.budget = cus;
-        const size_t part_bytes = (size_t)sc.budget * 128 * 128 * 4, cnt_bytes = split_count_bytes((int)sc.budget);
-        if (!(st = pool_alloc(&part, part_bytes + cnt_bytes, s))) {
-            sc.part = (float*)part;
-            sc.count = (int*)((char*)part + part_bytes);
-            st = launch_zero(sc.count, cnt_bytes, s);
-        }
-    }
-    if (!st) assign_split(cus, 1, dtype, tile, sc, sets, tile.m == 32 ? kSplitMinStagesKsw : kSplitMinStages);
-    PhaseArgs a;
-    std::memset(&a, 0, sizeof a);
-    a.alpha = 1.f;
-    a.beta = beta;
-    a.k_stagger = dtype == PCD_F32 ? 0 : auto_k_stagger(kp / stage_k(dtype, tile));
-    a.nt_store = (size_t)m * n * 4 >= kGemmNtBytes;
-    const int epi = mk_a ? (kn_b ? EPI_PLAIN_MKKN : EPI_PLAIN_MK) : (kn_b ? EPI_PLAIN_KN : EPI_PLAIN);
-    if (!st) st = launch_phase(dtype, tile, epi, sets[0], a, s);
-    release();
-    if (part) {
-        int st2 = pool_free(part, s);
-        if (!st) st = st2;
-    }
-    return st;
-}
-
-// Strided batched GEMM: C_i = A_i B_i for i < batch, row-major, A_i [m x k] at
-// dA + i m k, B_i [k x n] at dB + i k n, C_i [m x n] at dC + i m n.  Both
-// operands of every item are packed K-contiguous in one launch each; the
-// items are the problems of grouped phase launches (kMaxProblems per launch),
-// their tiles dealt over the XCDs together.
-static int gemm_batched_common(int dtype, const void* dA, const void* dB, float* dC, int batch, int m, int k, int n,
-                               void* stream_) {
-    if (!dA || !dB || !dC) return fail(PCD_INVALID_VALUE, "pcd_gemm_batched: null pointer");
     if (batch < 1 || m < 1 || k < 1 || n < 1)
-        return fail(PCD_INVALID_VALUE, "pcd_gemm_batched: bad shape %d x (%d x %d x %d)", batch, m, k, n);
+        return fail(PCD_INVALID_VALUE, "pcd_gemm: bad shape %d x (%d x %d x %d)", batch, m, k, n);
     hipStream_t s = (hipStream_t)stream_;
     int dev = 0, cus = 256;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const Tile tile = choose_gemm_tile(dtype, m, n, cus, batch);
-    const int mp = (int)round_up(m, tile.m), np = (int)round_up(n, tile.n), kp = (int)round_up(k, kFeatPad);
-    const int ob = op_bytes(dtype);
-    const size_t a_item = (size_t)mp * kp * ob, b_item = (size_t)np * kp * ob;
-    // Each B_i [k x n] is read where it lies (EPI_PLAIN_KN) when the tile has
-    // that form, its columns fill whole tiles, K is a whole number of stages and
-    // every item starts 16-byte aligned.
-    // (and not on the 128 x 128 tile when B_i is a quarter of A_i or smaller: see gemm_common)
-    const bool kn_b = kn_tile(ob, tile.m, tile.n, false) && n == np && k == kp && (uintptr_t)dB % 16 == 0 &&
-                      !(tile.m == 128 && (size_t)n * 4 <= (size_t)m);
-    void *pa = nullptr, *pb = nullptr;
-    int st = pool_alloc(&pa, a_item * batch, s);
-    if (!st && !kn_b) st = pool_alloc(&pb, b_item * batch, s);
-    auto pack = [&](const void* src, int rows, int cols, int trans, void* dst, int prow, int pcol) -> int {
-        const int grid = (int)std::min<size_t>(((size_t)batch * prow * pcol + 255) / 256, 16384);
+    const int ob = op_bytes(dtype), unit = 16 / ob;
+    const int kp = (int)round_up(k, stage_k(dtype, tile));
+    auto aligned = [&](const void* p, size_t item) {
+        return (uintptr_t)p % 16 == 0 && (batch == 1 || item * ob % 16 == 0);
+    };
+    // Except that the transposing reads cost the 16-bit 128 x 128 tile about a
+    // fifth of its time, more than packing an operand a quarter the other's size
+    // or smaller takes (512 x 8192 x 8192 bf16, A transposed: 0.089 ms in place,
+    // 0.081 packed; the other tiles lose 2-5% and read in place).
+    const bool small_a = ob == 2 && tile.m == 128 && (size_t)m * 4 <= (size_t)n;
+    const bool small_b = ob == 2 && tile.m == 128 && (size_t)n * 4 <= (size_t)m;
+    const bool whole_k = k == kp, kn = whole_k && kn_tile(ob, tile.m, tile.n, false);
+    const bool direct_a = whole_k && !trans_a && k % unit == 0 && aligned(dA, (size_t)m * k);
+    const bool direct_b = whole_k && trans_b && k % unit == 0 && aligned(dB, (size_t)k * n);
+    const bool mk_a = kn && trans_a && !small_a && m % unit == 0 && aligned(dA, (size_t)m * k);
+    const bool kn_b = kn && !trans_b && !small_b && n % unit == 0 && aligned(dB, (size_t)k * n);
+    void *pa = nullptr, *pb = nullptr, *part = nullptr;
+    auto pack = [&](const void* src, int rows, int trans, void* dst) -> int {
         const int f32 = dtype == PCD_F32;
         switch (dtype) {
-        case PCD_F32: hipLaunchKernelGGL(pack_batched_kernel<float>, dim3(grid), dim3(256), 0, s, src, f32, batch, rows, cols, trans, dst, prow, pcol); break;
-        case PCD_BF16: hipLaunchKernelGGL(pack_batched_kernel<bf16_t>, dim3(grid), dim3(256), 0, s, src, f32, batch, rows, cols, trans, dst, prow, pcol); break;
-        default: hipLaunchKernelGGL(pack_batched_kernel<f16_t>, dim3(grid), dim3(256), 0, s, src, f32, batch, rows, cols, trans, dst, prow, pcol); break;
+        case PCD_F32: pack_op<float>(s, src, f32, rows, k, trans, dst, rows, kp, kp, batch); break;
+        case PCD_BF16: pack_op<bf16_t>(s, src, f32, rows, k, trans, dst, rows, kp, kp, batch); break;
+        default: pack_op<f16_t>(s, src, f32, rows, k, trans, dst, rows, kp, kp, batch); break;
         }
-        return from_hip(hipGetLastError(), "pack_batched_kernel launch");
+        return from_hip(hipGetLastError(), "pack_kernel launch");
     };
-    // the kernel's A is A_i [m x k]; its B is B_i^T [n x k] (B_i read transposed)
-    if (!st) st = pack(dA, m, k, 0, pa, mp, kp);
-    if (!st && !kn_b) st = pack(dB, n, k, 1, pb, np, kp);
+    int st = PCD_SUCCESS;
+    if (!direct_a && !mk_a)
+        if (!(st = pool_alloc(&pa, (size_t)batch * m * kp * ob, s))) st = pack(dA, m, trans_a, pa);
+    if (!st && !direct_b && !kn_b)
+        if (!(st = pool_alloc(&pb, (size_t)batch * n * kp * ob, s))) st = pack(dB, n, !trans_b, pb);
+    std::vector<ProblemSet> sets(1);
+    std::memset(&sets[0], 0, sizeof(ProblemSet));
+    sets[0].n = 1;
+    Problem& p = sets[0].p[0];
+    p.A = pa ? pa : dA;
+    p.lda = mk_a ? m : kp;   // the row pitch of a transposed A, else of the K-contiguous rows
+    p.B = pb ? pb : dB;
+    p.ldb = kn_b ? n : kp;   // the row pitch of row-major B, else of the K-contiguous copy
+    p.M = m;
+    p.N = n;
+    p.K = kp;
+    p.tiles_m = (m + tile.m - 1) / tile.m;
+    p.tiles_n = (n + tile.n - 1) / tile.n;
+    p.tiles = p.tiles_m * p.tiles_n;
+    p.ldo = n;
+    p.m = dC;
+    // Split-K scratch from the pool; the counters start at zero (a fill
+    // kernel, so a captured call stays free of memset nodes).
+    if (!st && batch == 1 && tile.m * tile.n <= 128 * 128 && p.tiles * 2 <= cus) {
+        SplitScratch sc;
+        sc.budget = cus;
+        const size_t part_bytes = (size_t)sc.budget * 128 * 128 * 4, cnt_bytes = split_count_bytes((int)sc.budget);
+        if (!(st = pool_alloc(&part, part_bytes + cnt_bytes, s))) {
+            sc.part = (float*)part;
+            sc.count = (int*)((char*)part + part_bytes);
+            assign_split(cus, 1, dtype, tile, sc, sets, tile.m == 32 ? kSplitMinStagesKsw : kSplitMinStages);
+            if (p.ksplit > 1) st = launch_zero(sc.count, cnt_bytes, s);
+        }
+    }
     PhaseArgs a;
     std::memset(&a, 0, sizeof a);
     a.alpha = 1.f;
-    a.beta = 0.f;
+    a.beta = beta;
     a.k_stagger = dtype == PCD_F32 ? 0 : auto_k_stagger(kp / stage_k(dtype, tile));
     a.nt_store = (size_t)batch * m * n * 4 >= kGemmNtBytes;
-    for (int i0 = 0; i0 < batch && !st; i0 += kMaxProblems) {
-        ProblemSet ps;
-        std::memset(&ps, 0, sizeof ps);
-        ps.n = std::min(kMaxProblems, batch - i0);
-        for (int q = 0; q < ps.n; ++q) {
-            const size_t i = (size_t)(i0 + q);
-            Problem& p = ps.p[q];
-            p.A = (const char*)pa + i * a_item;
-            p.lda = kp;
-            p.B = kn_b ? (const void*)((const char*)dB + i * (size_t)k * n * ob) : (const void*)((const char*)pb + i * b_item);
-            p.ldb = kn_b ? n : kp;
-            p.M = m;
-            p.N = n;
-            p.K = kp;
-            p.tiles_m = mp / tile.m;
-            p.tiles_n = np / tile.n;
-            p.tiles = p.tiles_m * p.tiles_n;
-            p.ldo = n;
-            p.m = dC + i * (size_t)m * n;
+    a.item_tiles = p.tiles_m * p.tiles_n;
+    a.item_a = (size_t)m * kp * ob;
+    a.item_b = (size_t)n * kp * ob;
+    a.item_c = (size_t)m * n;
+    const int epi = mk_a ? (kn_b ? EPI_PLAIN_MKKN : EPI_PLAIN_MK) : (kn_b ? EPI_PLAIN_KN : EPI_PLAIN);
+    // Launches of at most 2^24 work units (one, but for batches of millions).
+    const int most = std::max(1, (1 << 24) / a.item_tiles);
+    for (int i0 = 0; i0 < batch && !st; i0 += most) {
+        a.items = std::min(most, batch - i0);
+        if (batch > 1) p.tiles = a.items * a.item_tiles;
+        st = launch_phase(dtype, tile, epi, sets[0], a, s);
+        p.A = (const char*)p.A + most * a.item_a;
+        p.B = (const char*)p.B + most * a.item_b;
+        p.m += most * a.item_c;
+    }
+    for (void* q : {pa, pb, part})
+        if (q) {
+            const int st2 = pool_free(q, s);
+            if (!st) st = st2;
         }
-        st = launch_phase(dtype, tile, kn_b ? EPI_PLAIN_KN : EPI_PLAIN, ps, a, s);
-    }
-    if (pa) {
-        int st2 = pool_free(pa, s);
-        if (!st) st = st2;
-    }
-    if (pb) {
-        int st2 = pool_free(pb, s);
-        if (!st) st = st2;
-    }
     return st;
+}
+
+// Strided batched products (MatMulBatchedDevice): A_i [m x k], B_i [k x n].
+static int gemm_batched_common(int dtype, const void* dA, const void* dB, float* dC, int batch, int m, int k, int n,
+                               void* stream) {
+    return gemm_common(dtype, dA, dB, dC, batch, m, k, n, 0, 0, 0.f, stream);
 }
 
 int pcd_gemm_f32_batched(const float* dA, const float* dB, float* dC, int batch, int m, int k, int n, void* stream) {
@@ -1728,17 +1670,17 @@ int pcd_gemm_f16_batched(const uint16_t* dA, const uint16_t* dB, float* dC, int 
 
 int pcd_gemm_f32(const float* dA, const float* dB, float* dC, int m, int k, int n, int trans_a, int trans_b,
                  float beta, void* stream) {
-    return gemm_common(PCD_F32, dA, dB, dC, m, k, n, trans_a, trans_b, beta, stream);
+    return gemm_common(PCD_F32, dA, dB, dC, 1, m, k, n, trans_a, trans_b, beta, stream);
 }
 
 int pcd_gemm_bf16(const uint16_t* dA, const uint16_t* dB, float* dC, int m, int k, int n, int trans_a, int trans_b,
                   float beta, void* stream) {
-    return gemm_common(PCD_BF16, dA, dB, dC, m, k, n, trans_a, trans_b, beta, stream);
+    return gemm_common(PCD_BF16, dA, dB, dC, 1, m, k, n, trans_a, trans_b, beta, stream);
 }
 
 int pcd_gemm_f16(const uint16_t* dA, const uint16_t* dB, float* dC, int m, int k, int n, int trans_a, int trans_b,
                  float beta, void* stream) {
-    return gemm_common(PCD_F16, dA, dB, dC, m, k, n, trans_a, trans_b, beta, stream);
+    return gemm_common(PCD_F16, dA, dB, dC, 1, m, k, n, trans_a, trans_b, beta, stream);
 }
 
 // ---------------------------------------------------------------- PC model
