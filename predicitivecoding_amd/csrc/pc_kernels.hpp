@@ -155,13 +155,11 @@ struct PhaseArgs {
     int act;
     float eta, act_reg;
     float alpha, beta;          // PLAIN
-    int items, item_tiles;      // PLAIN: products of the launch's one shape (<= 1: one) and the work units of each
-    size_t item_a, item_b, item_c;   // PLAIN: bytes from one product's A, B to the next, elements of its C
+    int shared_from;            // energy slots from this one on hold one row's energies, the same for every row
     float* energy_part;         // [nslots x ldp] per-row partial energies (nullable)
     int ldp, nslots;
     float* energy_out;          // UPDATE prologue: row energies of step t (nullable)
     int batch, t;
-    int shared_from;            // energy slots from this one on hold one row's energies, the same for every row
     const int* row_req;         // ragged: request of each row (nullable)
     const int* done_at;         // ragged: first step a request no longer runs
     int tile_order;             // TILE_INTERLEAVED or TILE_CONTIGUOUS (see phase_grid)
@@ -170,6 +168,8 @@ struct PhaseArgs {
     const int* act_count;       // ragged: their number
     int nt_store;               // settling epilogues store their full rows non-temporally
     int nt_load;                // settling epilogues load their fp32 state rows non-temporally
+    int items, item_tiles;      // PLAIN: products of the launch's one shape (<= 1: one) and the work units of each
+    size_t item_a, item_b, item_c;   // PLAIN: bytes from one product's A, B to the next, elements of its C
 };
 
 // How a phase's tiles are dealt over the XCDs.
@@ -917,7 +917,8 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     if (EPI == EPI_UPDATE && args.energy_out != nullptr) {
         for (int row = (vgrid - 1 - vblock) * C::NT + tid; row < args.batch; row += vgrid * C::NT) {
             gst(args.energy_out + (size_t)args.t * args.batch + row,
-                sum_slots(args.energy_part, args.ldp, args.nslots, row, args.shared_from));
+                sum_slots(args.energy_part, args.ldp, args.nslots, row,
+                          C::KSW || C::WD ? args.nslots : args.shared_from));   // (no one-row layers on those tiles)
         }
     }
 
@@ -1014,12 +1015,12 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // latency passes under the K sweep.
     f32x4 epi_state{}, epi_bias{};
     if constexpr (C::KW > 1 && (EPI == EPI_ERROR || EPI == EPI_UPDATE)) {
-        const size_t eidx = (size_t)(row0 + (lane & 31)) * P.ldi + col0 + 8 * wave + 4 * (lane >> 5);
+        const size_t eidx = (size_t)(row0 + (lane & 31)) * P.ldo + col0 + 8 * wave + 4 * (lane >> 5);
         if constexpr (EPI == EPI_ERROR) {
             epi_state = gld4(P.mlow + eidx);
             epi_bias = gld4(P.bias + col0 + 8 * wave + 4 * (lane >> 5));
         } else {
-            epi_state = gld4((P.eself != nullptr ? P.eself : P.mlow) + eidx);
+            epi_state = gld4((P.eself != nullptr ? P.eself : P.m) + eidx);
         }
     }
 
