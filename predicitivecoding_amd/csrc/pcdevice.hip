@@ -16,6 +16,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -2629,23 +2630,21 @@ int pcd_pc_model_get_weights(pcd_model* m, int layer, float* W_out, float* b_out
     if (W_out) {
         // One contiguous copy: HIP copies a pitched block to pageable host memory
         // row by row, about 7 us each (all weights of 784-256-256-10: 8.8 ms, now
-        // 0.14; of 1024-1024-1024-1024-256: 28.7 ms, now 0.91).  Padded rows are
-        // closed up on the device first.
+        // 0.14; of 1024-1024-1024-1024-256: 28.7 ms, now 0.91).  Padded rows come
+        // over with their padding and are closed up here; without host memory
+        // for that, the pitched copy.
         const void* src = m->dtype == PCD_F32 ? (const void*)m->W[layer] : (const void*)m->W32[layer];
         const size_t bytes = (size_t)lo * sz * 4;
-        void* tight = nullptr;
-        int st = PCD_SUCCESS;
-        if (m->P[layer] != sz) {
-            if ((st = pool_alloc(&tight, bytes, nullptr))) return st;
+        const size_t pitch = (size_t)m->P[layer];
+        if (pitch == (size_t)sz) {
+            HIP_TRY(sync_memcpy(W_out, src, bytes, hipMemcpyDeviceToHost));
+        } else if (std::unique_ptr<float[]> rows{new (std::nothrow) float[(size_t)lo * pitch]}) {
+            HIP_TRY(sync_memcpy(rows.get(), src, (size_t)lo * pitch * 4, hipMemcpyDeviceToHost));
+            for (int r = 0; r < lo; ++r) std::memcpy(W_out + (size_t)r * sz, rows.get() + r * pitch, (size_t)sz * 4);
+        } else {
             std::lock_guard<std::mutex> no_capture(legacy_stream_mu());
-            st = copy_out_rows((float*)tight, sz, (const float*)src, m->P[layer], lo, nullptr);
+            HIP_TRY(hipMemcpy2D(W_out, (size_t)sz * 4, src, pitch * 4, (size_t)sz * 4, lo, hipMemcpyDeviceToHost));
         }
-        if (!st) st = from_hip(sync_memcpy(W_out, tight ? tight : src, bytes, hipMemcpyDeviceToHost), "weight copy");
-        if (tight) {
-            const int st2 = pool_free(tight, nullptr);
-            if (!st) st = st2;
-        }
-        if (st) return st;
     }
     if (b_out) HIP_TRY(sync_memcpy(b_out, m->bias[layer], (size_t)lo * 4, hipMemcpyDeviceToHost));
     return PCD_SUCCESS;
