@@ -493,7 +493,7 @@ long error_phase_tiles(const pcd_model* m, int batch, Tile t) {
 // runs four times as fast, and by the epilogue, which it splits over the
 // waves (784-256-256-10 at a batch of 64: fp32 +88%, bf16 +34%), unless the
 // fp32 persistent form, built on 64 x 64, is asked for.
-Tile choose_tile(const pcd_model* m, int batch) {
+Tile choose_tile(const pcd_model* m, int batch, int f32_tiles_per_cu = 1) {
     if (m->tile_m > 0) return Tile{m->tile_m, m->tile_n};
     const bool have_direct = m->direct && !m->Wpk.empty() && m->Wpk[1];
     if (m->direct == 2 && have_direct && batch <= 64) return Tile{64, 128, true};   // forced (option)
@@ -515,7 +515,8 @@ Tile choose_tile(const pcd_model* m, int batch) {
     // layers at 1024 rows (256 such tiles) 6.65 ms with 64 x 64 tiles, 6.07 with
     // 128 x 128; 3000-1500-700-300 at 768 rows (252) 2.06 and 2.14, at 1024 (336)
     // 2.47 and 2.21.
-    if (error_phase_tiles(m, batch, Tile{128, 128}) >= (m->dtype == PCD_F32 ? m->cus : want)) return Tile{128, 128};
+    if (error_phase_tiles(m, batch, Tile{128, 128}) >= (m->dtype == PCD_F32 ? (long)f32_tiles_per_cu * m->cus : want))
+        return Tile{128, 128};
     return Tile{64, 64};
 }
 
@@ -857,8 +858,8 @@ void build_phase_sets(const pcd_model* m, const Workspace* w, int batch, Tile ti
 // direct-weight one (and any batch of one row tile) a layer's single row takes
 // as long as its whole batch.  Elsewhere it was never slower: 0.995 to 1.42
 // times as fast over 72 networks and batches (128 to 4096 rows, fp32 and bf16).
-bool use_front(const pcd_model* m, const RelaxSpec& r) {
-    return m->shared_rows && m->L > 2 && !r.clamp_top && !r.keep_hidden && !r.persistent && r.row_req == nullptr &&
+bool use_front(const pcd_model* m, const Workspace* w, const RelaxSpec& r) {
+    return m->shared_rows && !w->Mr.empty() && m->L > 2 && !r.clamp_top && !r.keep_hidden && !r.persistent && r.row_req == nullptr &&
            r.tile.m >= 64 && !r.tile.wd && r.batch > r.tile.m;
 }
 
@@ -1004,7 +1005,7 @@ int enqueue_relax(pcd_model* m, Workspace* w, const RelaxSpec& r, hipStream_t s,
     const int batch = r.batch;
     const Tile tile = r.tile;
     int st;
-    const bool front = use_front(m, r);
+    const bool front = use_front(m, w, r);
     ZeroBatch zb;
     // with `front` the rows the layers share are the only states read before they are written
     if (front && (st = zb.add(w->Mr[1], front_row_bytes(m), s))) return st;
@@ -1989,7 +1990,7 @@ int scratch_device(int device, ScratchDevice** out) {
 // then split-K scratch for exactly the partial tiles this call's phases use
 // (the split plan itself is the allocating path's, so the kernels and their
 // results are the same).  Returns the bytes the layout spans.
-size_t carve_workspace(const pcd_model* m, char* base, int batch, Tile tile, Workspace& w) {
+size_t carve_workspace(const pcd_model* m, char* base, int batch, Tile tile, bool front_rows, Workspace& w) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
         char* p = base + off;
@@ -2009,7 +2010,8 @@ size_t carve_workspace(const pcd_model* m, char* base, int batch, Tile tile, Wor
         if (l >= 1) w.D[l] = take(cap * m->P[l - 1] * ob);
         if (l >= 1 && l <= L - 2) w.E[l] = (float*)take(cap * m->P[l] * 4);
     }
-    carve_front_rows(m, &w, take(front_row_bytes(m)));
+    w.Mr.clear();
+    if (front_rows) carve_front_rows(m, &w, take(front_row_bytes(m)));
     w.slots_cap = energy_slots(m, tile);
     w.energy_part = (float*)take((size_t)w.slots_cap * cap * 4);
     w.split_count = (int*)take(split_count_bytes(m));
@@ -2052,10 +2054,17 @@ int pcd_pc_relax_noalloc(pcd_model* m, const float* x0, int batch, int steps, fl
     HIP_TRY(hipStreamIsCapturing(s, &cs));
     const bool capturing = cs != hipStreamCaptureStatusNone;
     if (!capturing && sd->recorded) HIP_TRY(hipStreamWaitEvent(s, sd->done, 0));
-    const Tile tile = choose_tile(m, batch);
+    Tile tile = choose_tile(m, batch);
     Workspace w;
     w.stream = s;
-    const size_t need = carve_workspace(m, base, batch, tile, w);
+    size_t need = carve_workspace(m, base, batch, tile, m->shared_rows, w);
+    // Near the array's end: without the rows the layers share, then (fp32) with
+    // the 128 x 128 tile only where it fills each CU twice, whose update phases
+    // need no split-K partials where the 64 x 64 tile's need none.
+    for (int per_cu = 1; need > kNoAllocScratchBytes && per_cu <= 2; ++per_cu) {
+        tile = choose_tile(m, batch, per_cu);
+        need = carve_workspace(m, base, batch, tile, false, w);
+    }
     if (need > kNoAllocScratchBytes)
         return fail(PCD_INVALID_VALUE,
                     "pcd_pc_relax_noalloc: %d rows of this model need %zu bytes of scratch, beyond its %zu; use "

@@ -97,6 +97,32 @@ def test_noalloc_refuses_a_batch_beyond_its_scratch():
         model.close()
 
 
+@pytest.mark.parametrize("sizes,batch", [([8192, 4096, 4096, 4096, 4096, 1024], 100), ([2048, 64, 64, 10], 3300)])
+def test_noalloc_takes_what_fits_its_scratch_without_extras(sizes, batch):
+    """The rows that unreached layers share, and the split-K partials of a large tile, are left out where they do not
+    fit: a settling whose own states and deltas do is taken.  (First case: layer 0 narrowed until less than one 64-wide
+    step of it is free, which the shared rows, about 250 KB, do not fit.  Second: 61.5 MB of states and deltas.)"""
+    import re
+
+    from predicitivecoding_amd.errors import DeviceException
+    x = make_inputs(batch, sizes[0], seed=5)
+    if batch == 100:
+        model = _model(sizes, 1, "f32", 0, 0.1, seed=0)
+        model.set_option("shared_rows", 0)
+        with pytest.raises(DeviceException, match="bytes of scratch") as e:
+            _run("pcd_pc_relax_noalloc", model, x, 4)
+        need = int(re.search(r"need (\d+) bytes", str(e.value)).group(1))
+        step = 256 * 4 * (2 * 64 + 1)   # 256 padded rows: state, delta, energy slot of 64 columns
+        sizes = [sizes[0] - 64 * -(-(need - (64 << 20)) // step)] + sizes[1:]
+        x = np.ascontiguousarray(x[:, :sizes[0]])
+        model.close()
+    model = _model(sizes, 1, "f32", 0, 0.1, seed=0)
+    got, want = (_run(fn, model, x, 4) for fn in ("pcd_pc_relax_noalloc", "pcd_pc_relax"))
+    for a, b in zip(got, want):   # fp32 sums of up to 8192 products in another order
+        assert np.max(np.abs(a - b) / (1 + np.abs(b))) <= 1e-5
+    model.close()
+
+
 def test_noalloc_calls_on_two_streams_are_ordered():
     # Two models' calls queued back to back on two streams, with no
     # synchronisation between them, share the device's one scratch array: the
