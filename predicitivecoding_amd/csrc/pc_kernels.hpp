@@ -1519,11 +1519,12 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // (1024-wide fp32 network), -5% on a whole classification settling.
     if (ks > 1) {
         const int tile = local;
-        // Lane-contiguous layout: block (i, j) of this wave holds each lane's 16
-        // accumulators as 8 consecutive 64-bit pairs (a wave's block is 4 KB).
+        // Block (i, j) of this wave is 4 KB: 64-bit pair q of a lane's 16
+        // accumulators is word q * 64 + lane, so one access of the wave is 512
+        // consecutive bytes.
         typedef unsigned long long u64;
         gu64* part = (gu64*)(P.part + (size_t)tile * ks * (BM * BN));   // global, not flat: see flush_block
-        auto slot_of = [&](int i, int j) PCD_INLINE { return (((wmn * C::FM + i) * C::FN + j) * 64 + lane) * 8; };
+        auto slot_of = [&](int i, int j) PCD_INLINE { return ((wmn * C::FM + i) * C::FN + j) * 512 + lane; };
         constexpr int UNIT = BM * BN / 2;   // 64-bit words of one partial tile
         gu64* mine = part + (size_t)split * UNIT;
         if (writer) {
@@ -1534,7 +1535,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
                         constexpr int q = decltype(Q)::value;
                         const u64 w =
                             (u64)__float_as_uint(acc[i][j][2 * q]) | ((u64)__float_as_uint(acc[i][j][2 * q + 1]) << 32);
-                        __hip_atomic_store(mine + slot_of(i, j) + q, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(mine + slot_of(i, j) + q * 64, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     });
                 });
             });
@@ -1565,7 +1566,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
                             if (k < ks && k != split)
                                 static_for<0, 8>([&](auto Q) PCD_INLINE {
                                     pv[decltype(K)::value][decltype(Q)::value] =
-                                        __hip_atomic_load(part + (size_t)k * UNIT + slot_of(i, j) + decltype(Q)::value,
+                                        __hip_atomic_load(part + (size_t)k * UNIT + slot_of(i, j) + decltype(Q)::value * 64,
                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                                 });
                         });
