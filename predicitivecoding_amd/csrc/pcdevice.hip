@@ -485,15 +485,15 @@ long error_phase_tiles(const pcd_model* m, int batch, Tile t) {
 }
 
 // The largest tile that still gives every CU at least two workgroups per
-// phase (a phase with fewer tiles leaves SIMDs idle), or, in fp32, one of
-// 128 x 128.  256 x 256 only for 16-bit
+// phase (a phase with fewer tiles leaves SIMDs idle); in fp32 fewer of 128 x 128
+// too (see there; `f32_two_per_cu`: not).  256 x 256 only for 16-bit
 // operands with every layer at least 1024 wide.  A settling whose error
 // phase has fewer 64 x 64 tiles than the GPU has CUs takes the K-shared
 // 32 x 32 tile: its phases are bound by one tile's K sweep, which that tile
 // runs four times as fast, and by the epilogue, which it splits over the
 // waves (784-256-256-10 at a batch of 64: fp32 +88%, bf16 +34%), unless the
 // fp32 persistent form, built on 64 x 64, is asked for.
-Tile choose_tile(const pcd_model* m, int batch, int f32_tiles_per_cu = 1) {
+Tile choose_tile(const pcd_model* m, int batch, bool f32_two_per_cu = false) {
     if (m->tile_m > 0) return Tile{m->tile_m, m->tile_n};
     const bool have_direct = m->direct && !m->Wpk.empty() && m->Wpk[1];
     if (m->direct == 2 && have_direct && batch <= 64) return Tile{64, 128, true};   // forced (option)
@@ -510,13 +510,27 @@ Tile choose_tile(const pcd_model* m, int batch, int f32_tiles_per_cu = 1) {
         for (int l = 0; l < m->L; ++l) wide = wide && m->s[l] >= 1024;
         if (wide && error_phase_tiles(m, batch, Tile{256, 256}) >= want) return Tile{256, 256};
     }
-    // fp32: one 128 x 128 tile per CU is enough, since that tile multiplies in
-    // split bf16 (split3_tile) at 1.4 times the fp32 MFMAs' rate: 1024-wide
-    // layers at 1024 rows (256 such tiles) 6.65 ms with 64 x 64 tiles, 6.07 with
-    // 128 x 128; 3000-1500-700-300 at 768 rows (252) 2.06 and 2.14, at 1024 (336)
-    // 2.47 and 2.21.
-    if (error_phase_tiles(m, batch, Tile{128, 128}) >= (m->dtype == PCD_F32 ? (long)f32_tiles_per_cu * m->cus : want))
-        return Tile{128, 128};
+    const long t128 = error_phase_tiles(m, batch, Tile{128, 128});
+    if (t128 >= want) return Tile{128, 128};
+    // fp32: one 128 x 128 tile per CU is enough where the K sweeps (`mean_k` over
+    // both phases' tiles) pay its start and few of its rows are padding, since it
+    // multiplies in split bf16 (split3_tile) at 1.4 times the fp32 MFMAs' rate:
+    // 1024-wide layers at 1024 rows (256 such tiles) 6.65 ms with 64 x 64 tiles,
+    // 6.07 with 128 x 128, at 1600 rows 1.87 and 1.70 (10 steps); 3000-1500-700-300
+    // at 1024 (336) 2.42 and 2.11; but 500-wide layers at 3000 rows 0.97 and 1.02,
+    // 4096-wide ones at 260 5.22 and 5.31.  Long sweeps pay for it with idle CUs
+    // too, against three 64 x 64 tiles on a CU: 192 tiles, 4096-wide at 200 rows
+    // 4.02 and 3.64, 2048-wide at 500 2.09 and 1.98; 1024-wide at 700 1.09 and 1.16.
+    if (m->dtype == PCD_F32 && !f32_two_per_cu && 4L * batch >= 3 * (long)round_up(batch, 128)) {
+        double macs = 0, cols = 0;
+        for (int l = 1; l < m->L; ++l) {
+            macs += 2.0 * m->s[l] * m->s[l - 1];
+            cols += (double)m->s[l] + m->s[l - 1];
+        }
+        const double mean_k = macs / cols;
+        if (mean_k >= 640 && t128 >= m->cus) return Tile{128, 128};
+        if (mean_k >= 2048 && error_phase_tiles(m, batch, Tile{64, 64}) > want) return Tile{128, 128};
+    }
     return Tile{64, 64};
 }
 
@@ -1519,7 +1533,16 @@ int pcd_event_elapsed_ms(float* ms, void* start, void* end) {
 // Output tile of a provider GEMM: 256 x 256 (16-bit operands) while it still
 // gives every CU a tile, then 128 x 128 while that does, else 64 x 64 (whose
 // few tiles split-K then spreads over the CUs); fp32 products with fewer
-// 64 x 64 tiles than CUs take the K-shared 32 x 32 tile.  `batch` products of
+// 64 x 64 tiles than CUs take the K-shared 32 x 32 tile.
+// With fewer 128 x 128 tiles than CUs that tile is still the faster one where
+// some CU would get a third 64 x 64 tile and K is long enough to pay its start
+// (64 x 64 -> 128 x 128: 1300 x 3000 x 2000 bf16 51.6 -> 45.9 us, fp32 171 -> 146;
+// 1700 x 600 x 1500 25.2 -> 24.8 and 49.8 -> 47.4; 1600 x 512 x 1600 12.2 -> 13.1
+// and 32 -> 33 to 36), and in fp32, where it multiplies at 1.4 times the other
+// tiles' rate, wherever K ranges of 1024 and more spread it over the CUs (1024 x
+// 4096 x 1024 90 -> 66 us, 256 x 8192 x 4096 181 -> 117, 640 x 8192 x 640 95 ->
+// 67; ranges of 400 lose: 300 x 2048 x 2048 33 -> 36).  Error against 64 bits
+// falls there (K = 4096: 5.7e-7 -> 1.9e-7).  `batch` products of
 // the same shape count together, but only among the tiles that fit one
 // product: a tile wider than the product (rounded up to 64) in either
 // dimension would be mostly padding, in MFMA work and in packed operand
@@ -1528,11 +1551,17 @@ int pcd_event_elapsed_ms(float* ms, void* start, void* end) {
 // stored non-temporally: a caller reads them long after the L2 has turned over.
 constexpr size_t kGemmNtBytes = (size_t)64 << 20;
 
-static Tile choose_gemm_tile(int dtype, int m, int n, int cus, int batch = 1) {
+static Tile choose_gemm_tile(int dtype, int m, int k, int n, int cus, int batch = 1) {
     auto tiles = [&](int t) { return (long)batch * ((m + t - 1) / t) * ((n + t - 1) / t); };
     auto fits = [&](int t) { return t <= (int)round_up(m, 64) && t <= (int)round_up(n, 64); };
     if (dtype != PCD_F32 && fits(256) && tiles(256) >= cus) return Tile{256, 256};
     if (fits(128) && tiles(128) >= cus) return Tile{128, 128};
+    if (fits(128) && 4L * m * n * batch >= 3L * tiles(128) * 128 * 128) {   // at most a quarter of it padding
+        if (k >= 640 && tiles(64) > 2L * cus) return Tile{128, 128};
+        const long split = std::min<long>(kMaxSplit, cus / tiles(128));
+        if (dtype == PCD_F32 && batch == 1 && tiles(128) * split * 4 >= 3L * cus && k / split >= 1024)
+            return Tile{128, 128};
+    }
     if (dtype == PCD_F32 && tiles(64) < cus) return Tile{32, 32};
     return Tile{64, 64};
 }
@@ -1560,7 +1589,7 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     int dev = 0, cus = 256;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const Tile tile = choose_gemm_tile(dtype, m, n, cus, batch);
+    const Tile tile = choose_gemm_tile(dtype, m, k, n, cus, batch);
     const int ob = op_bytes(dtype), unit = 16 / ob;
     const int kp = (int)round_up(k, stage_k(dtype, tile));
     auto aligned = [&](const void* p, size_t item) {
@@ -1608,6 +1637,26 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     p.tiles = p.tiles_m * p.tiles_n;
     p.ldo = n;
     p.m = dC;
+    // fp32 128 x 128 tiles for less than every CU, but more than half of them:
+    // the K ranges per tile (up to 4, of at least 1024) that leave the CUs the
+    // shortest sweep, an exchange costing about a hundredth of one.  1536 x 8192
+    // x 1536 (144 tiles): 372 us whole, 273 in four ranges.
+    const int t128 = dtype == PCD_F32 && batch == 1 && tile.m == 128 ? p.tiles : 0;
+    if (!st && t128 * 2 > cus && t128 < cus) {
+        auto cost = [&](int r) { return (double)((t128 * r + cus - 1) / cus) / r + 0.01 * r; };
+        int ks = 1;
+        for (int r = 2; r <= 4 && k / r >= 1024; ++r)
+            if (cost(r) < cost(ks)) ks = r;
+        const size_t part_bytes = (size_t)t128 * ks * 128 * 128 * 4, cnt_bytes = round_up((size_t)t128 * 4, 16);
+        // without scratch for it the product is not split
+        if (ks > 1 && pool_alloc(&part, part_bytes + cnt_bytes, s) == PCD_SUCCESS) {
+            p.part = (float*)part;
+            p.count = (int*)((char*)part + part_bytes);
+            p.ksplit = ks;
+            p.tiles = t128 * ks;
+            st = launch_zero(p.count, cnt_bytes, s);
+        }
+    }
     // Split-K scratch from the pool; the counters start at zero (a fill
     // kernel, so a captured call stays free of memset nodes).
     if (!st && batch == 1 && tile.m * tile.n <= 128 * 128 && p.tiles * 2 <= cus) {
@@ -2061,8 +2110,9 @@ int pcd_pc_relax_noalloc(pcd_model* m, const float* x0, int batch, int steps, fl
     // Near the array's end: without the rows the layers share, then (fp32) with
     // the 128 x 128 tile only where it fills each CU twice, whose update phases
     // need no split-K partials where the 64 x 64 tile's need none.
-    for (int per_cu = 1; need > kNoAllocScratchBytes && per_cu <= 2; ++per_cu) {
-        tile = choose_tile(m, batch, per_cu);
+    for (bool two : {false, true}) {
+        if (need <= kNoAllocScratchBytes) break;
+        tile = choose_tile(m, batch, two);
         need = carve_workspace(m, base, batch, tile, false, w);
     }
     if (need > kNoAllocScratchBytes)
