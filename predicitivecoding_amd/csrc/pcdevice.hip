@@ -791,18 +791,6 @@ struct RelaxSpec {
     float* last_energy = nullptr;
 };
 
-// The split-K plan of both phases of a step.
-void assign_phase_splits(const pcd_model* m, const Workspace* w, Tile tile, std::vector<ProblemSet>& err,
-                         std::vector<ProblemSet>& upd) {
-    SplitScratch sc;
-    sc.part = w->split_part;
-    sc.count = w->split_count;
-    sc.budget = split_part_tiles(m);
-    const int smin = m->split_min > 0 ? m->split_min : tile.m == 32 ? kSplitMinStagesKsw : kSplitMinStages;
-    assign_split(m->cus, m->split_k, m->dtype, tile, sc, err, smin);
-    assign_split(m->cus, m->split_k, m->dtype, tile, sc, upd, smin);
-}
-
 // Problem sets of the two phases for a batch; problems beyond kMaxProblems
 // spill into further sets (still one phase: the problems are independent).
 void build_phase_sets(const pcd_model* m, const Workspace* w, int batch, Tile tile, int clamp_top,
@@ -861,7 +849,13 @@ void build_phase_sets(const pcd_model* m, const Workspace* w, int batch, Tile ti
         p.mop = m->dtype == PCD_F32 ? nullptr : w->S[l];
         p.eself = l <= L - 2 ? w->E[l] : nullptr;
     }
-    assign_phase_splits(m, w, tile, err, upd);
+    SplitScratch sc;
+    sc.part = w->split_part;
+    sc.count = w->split_count;
+    sc.budget = split_part_tiles(m);
+    const int smin = m->split_min > 0 ? m->split_min : tile.m == 32 ? kSplitMinStagesKsw : kSplitMinStages;
+    assign_split(m->cus, m->split_k, m->dtype, tile, sc, err, smin);
+    assign_split(m->cus, m->split_k, m->dtype, tile, sc, upd, smin);
     *nslots = slot;
 }
 
@@ -890,8 +884,12 @@ bool use_front(const pcd_model* m, const Workspace* w, const RelaxSpec& r) {
 //          l  = t + 1   Delta_l per sample, X_l (or the top's M_l) from the
 //                       shared row (ldi = 0): the layer becomes per-sample
 //          l  > t + 1   one row
-// From step L - 1 on every layer is per sample.  The values are those of the
-// general sets, sample by sample.  Of a settling of L layers and T >= L - 1
+// From step L - 1 on every layer is per sample.  A one-row problem keeps the K
+// ranges of the general sets' problem, so its sums are the general sets' (but
+// for the row tile's K stagger: it has row tile 0's), they match the unsplit
+// feed-forward sweep's wherever the general ones do (a warm start's errors are
+// then exactly zero), and its partial tiles are some of the general problem's:
+// whatever scratch holds the general sets' partials holds these.  Of a settling of L layers and T >= L - 1
 // steps this leaves 2T(L-1) - (L-2)(L-1) problems of the batch's size.  12 x
 // 8192 bf16 at 8192 rows, T = 16 (242 of 352 problems): 308.7 -> 218.2 ms; 6 x
 // 4096 at 4096 rows, T = 32 (300 of 320): 41.9 -> 40.1 ms; 8 x 512 fp32 at 600
@@ -904,7 +902,7 @@ void build_front_sets(const pcd_model* m, const Workspace* w, int batch, Tile ti
     auto one_row = [](Problem& p) {
         p.M = 1;
         p.tiles_m = 1;
-        p.tiles = p.tiles_n;
+        p.tiles = p.tiles_n * p.ksplit;
         p.lda = 0;
     };
     int l = 1;
@@ -935,7 +933,6 @@ void build_front_sets(const pcd_model* m, const Workspace* w, int batch, Tile ti
             p.m = w->Mr[l];
             if (p.mop) p.mop = w->Sr[l];
         }
-    assign_phase_splits(m, w, tile, err, upd);
 }
 
 int auto_k_stagger(int nk, bool one_row_tile) {
@@ -2078,6 +2075,22 @@ size_t carve_workspace(const pcd_model* m, char* base, int batch, Tile tile, boo
     return round_up(end, 256);
 }
 
+// The tile and layout of an allocation-free settling from `base`; the bytes
+// they span, more than kNoAllocScratchBytes if nothing fits.  Near the array's
+// end: without the rows the layers share, then (fp32) with the 128 x 128 tile
+// only where it fills each CU twice, whose update phases need no split-K
+// partials where the 64 x 64 tile's need none.
+size_t plan_noalloc(const pcd_model* m, char* base, int batch, Tile* tile, Workspace& w) {
+    *tile = choose_tile(m, batch);
+    size_t need = carve_workspace(m, base, batch, *tile, m->shared_rows, w);
+    for (bool two : {false, true}) {
+        if (need <= kNoAllocScratchBytes) break;
+        *tile = choose_tile(m, batch, two);
+        need = carve_workspace(m, base, batch, *tile, false, w);
+    }
+    return need;
+}
+
 }  // namespace
 
 extern "C" {
@@ -2103,18 +2116,10 @@ int pcd_pc_relax_noalloc(pcd_model* m, const float* x0, int batch, int steps, fl
     HIP_TRY(hipStreamIsCapturing(s, &cs));
     const bool capturing = cs != hipStreamCaptureStatusNone;
     if (!capturing && sd->recorded) HIP_TRY(hipStreamWaitEvent(s, sd->done, 0));
-    Tile tile = choose_tile(m, batch);
     Workspace w;
     w.stream = s;
-    size_t need = carve_workspace(m, base, batch, tile, m->shared_rows, w);
-    // Near the array's end: without the rows the layers share, then (fp32) with
-    // the 128 x 128 tile only where it fills each CU twice, whose update phases
-    // need no split-K partials where the 64 x 64 tile's need none.
-    for (bool two : {false, true}) {
-        if (need <= kNoAllocScratchBytes) break;
-        tile = choose_tile(m, batch, two);
-        need = carve_workspace(m, base, batch, tile, false, w);
-    }
+    Tile tile;
+    const size_t need = plan_noalloc(m, base, batch, &tile, w);
     if (need > kNoAllocScratchBytes)
         return fail(PCD_INVALID_VALUE,
                     "pcd_pc_relax_noalloc: %d rows of this model need %zu bytes of scratch, beyond its %zu; use "
