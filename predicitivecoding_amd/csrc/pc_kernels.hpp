@@ -1282,6 +1282,8 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     };
     const int c0 = wk * C::NCW;   // this wave's first chunk of a stage
     bool op_mfmas = true;   // the sweep on the operand type's own MFMAs
+    // fp32 in bf16 pieces: the first sweep's elements where there is a second.
+    f32x16 first[SPLIT3 ? C::FM : 1][SPLIT3 ? C::FN : 1];
     if constexpr (SPLIT3) {
         // Step kt (stage kt, 16 K elements of every row): the products of A's
         // first block row, then of its second.  One set of A's pieces is enough
@@ -1396,71 +1398,91 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         }
         if (kt < nk) step(I0, kt);
         static_for<0, 4>([&](auto X) PCD_INLINE { accs[0][decltype(X)::value / 2][decltype(X)::value % 2] += small[decltype(X)::value / 2][decltype(X)::value % 2]; });
-        // A result that is not finite: an operand was not (its pieces mix
+        // An element that is not finite: an operand was not (its pieces mix
         // infinities and NaNs), it rounded up to infinity as a bf16, or the sum
-        // overflowed.  The tile then takes the whole sweep again on the fp32
-        // MFMAs, which give their own infinities and NaNs.
-        // (A settling's rows past M hold what earlier calls left there and do not
-        // count.)
-        bool bad = false;
+        // overflowed.  Such elements take the values of a second sweep, on the
+        // fp32 MFMAs, which give their own infinities and NaNs; the tile's other
+        // elements keep theirs, so what a row gets does not depend on the rows
+        // beside it.  Rows that are not stored do not ask for that sweep (a
+        // settling's rows past M hold what earlier calls left there, and a
+        // ragged settling's rows that have left keep their states).
+        bool again = false;
         static_for<0, C::FM>([&](auto I) PCD_INLINE {
+            constexpr int i = decltype(I)::value;
+            bool bad = false;
             static_for<0, C::FN>([&](auto J) PCD_INLINE {
                 static_for<0, 16>([&](auto R) PCD_INLINE {
-                    constexpr int i = decltype(I)::value, j = decltype(J)::value, r = decltype(R)::value;
-                    bad |= (!TRM || row0 + wm * C::WTM + i * 32 + lr < P.M) &&
-                           !(fabsf(accs[0][i][j][r]) <= 3.402823466e38f);
+                    bad |= !(fabsf(accs[0][i][decltype(J)::value][decltype(R)::value]) <= 3.402823466e38f);
                 });
             });
+            const int row = row0 + wm * C::WTM + i * 32 + lr;
+            if (TRM && bad) bad = row < P.M && row_active(args, row);
+            again |= bad;
         });
         volatile __attribute__((address_space(3))) int* flag = (volatile __attribute__((address_space(3))) int*)smem;
         __syncthreads();   // every wave is done reading the stage ring
         if (tid == 0) *flag = 0;
         __syncthreads();
-        if (bad) *flag = 1;
+        if (again) *flag = 1;
         __syncthreads();
         op_mfmas = *flag != 0;
         if (op_mfmas) {
             __syncthreads();
             static_for<0, C::FM>([&](auto I) PCD_INLINE {
-                static_for<0, C::FN>([&](auto J) PCD_INLINE { accs[0][decltype(I)::value][decltype(J)::value] = f32x16{}; });
+                static_for<0, C::FN>([&](auto J) PCD_INLINE {
+                    constexpr int i = decltype(I)::value, j = decltype(J)::value;
+                    first[i][j] = accs[0][i][j];
+                    accs[0][i][j] = f32x16{};
+                });
             });
         }
     }
     if (op_mfmas) {
-    for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
-    stage_ready(0);
-    read_frags(0, c0, fa[0], fb[0]);
-    // Chunk c's MFMAs run while chunk c+1's fragments are read; the last chunk
-    // of a stage runs after the barrier that publishes the next stage, whose
-    // first fragments it overlaps.  The last stage is peeled off.
-    for (int kt = 0; kt + 1 < nk; ++kt) {
-        if (kt + C::D < nk) issue_stage(kt + C::D);
-        if constexpr (NC == 1) {
-            // One chunk per wave and stage (the K-shared tile on 16-bit
-            // operands): its MFMA runs across the barrier, and the next
-            // stage's fragments are read into the same registers after it.
-            mfmas(fa[0], fb[0]);
-            stage_ready(kt + 1);
-            read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
-        } else {
-            static_for<0, NC>([&](auto Cc) PCD_INLINE {
-                constexpr int c = decltype(Cc)::value;
-                if constexpr (c + 1 < NC) {
-                    read_frags(kt % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
-                } else {
-                    stage_ready(kt + 1);
-                    read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
-                }
-                mfmas(fa[c & 1], fb[c & 1]);
-                interleave();
+        for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
+        stage_ready(0);
+        read_frags(0, c0, fa[0], fb[0]);
+        // Chunk c's MFMAs run while chunk c+1's fragments are read; the last chunk
+        // of a stage runs after the barrier that publishes the next stage, whose
+        // first fragments it overlaps.  The last stage is peeled off.
+        for (int kt = 0; kt + 1 < nk; ++kt) {
+            if (kt + C::D < nk) issue_stage(kt + C::D);
+            if constexpr (NC == 1) {
+                // One chunk per wave and stage (the K-shared tile on 16-bit
+                // operands): its MFMA runs across the barrier, and the next
+                // stage's fragments are read into the same registers after it.
+                mfmas(fa[0], fb[0]);
+                stage_ready(kt + 1);
+                read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
+            } else {
+                static_for<0, NC>([&](auto Cc) PCD_INLINE {
+                    constexpr int c = decltype(Cc)::value;
+                    if constexpr (c + 1 < NC) {
+                        read_frags(kt % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
+                    } else {
+                        stage_ready(kt + 1);
+                        read_frags((kt + 1) % C::NS, c0, fa[0], fb[0]);
+                    }
+                    mfmas(fa[c & 1], fb[c & 1]);
+                    interleave();
+                });
+            }
+        }
+        static_for<0, NC>([&](auto Cc) PCD_INLINE {
+            constexpr int c = decltype(Cc)::value;
+            if constexpr (c + 1 < NC) read_frags((nk - 1) % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
+            mfmas(fa[c & 1], fb[c & 1]);
+        });
+        if constexpr (SPLIT3) {
+            static_for<0, C::FM>([&](auto I) PCD_INLINE {
+                static_for<0, C::FN>([&](auto J) PCD_INLINE {
+                    static_for<0, 16>([&](auto R) PCD_INLINE {
+                        constexpr int i = decltype(I)::value, j = decltype(J)::value, r = decltype(R)::value;
+                        const float v = first[i][j][r];
+                        if (fabsf(v) <= 3.402823466e38f) accs[0][i][j][r] = v;
+                    });
+                });
             });
         }
-    }
-    static_for<0, NC>([&](auto Cc) PCD_INLINE {
-        constexpr int c = decltype(Cc)::value;
-        if constexpr (c + 1 < NC) read_frags((nk - 1) % C::NS, c0 + c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
-        mfmas(fa[c & 1], fb[c & 1]);
-    });
     }
     }   // LDS-operand main loop
     static_for<1, NSPLIT>([&](auto Kc) PCD_INLINE {
