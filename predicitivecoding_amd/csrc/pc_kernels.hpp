@@ -295,13 +295,23 @@ template <> __device__ __forceinline__ void mfma_chunk<f16_t>(f32x16& acc, const
 
 // fp32 operands on the 128 x 128 tile: each fragment is split in registers into
 // three bf16 ones whose sum it is exactly (three round-to-nearest bf16 hold 24
-// bits and more): h = bf16(x), m = bf16(x - h), l = x - h - m.  The product of
-// two such fragments is l h + h l + m m + m h + h m + h h on the bf16 matrix
-// cores, summed in fp32, h h apart from the five small ones; the three terms
-// left out are below 2^-26 |x y|.  Six 32x32x16 bf16 MFMAs (192 cycles)
+// bits and more): h = bf16(x), m = bf16(x - h), l = x - h - m.  Not an element
+// below 2^-109, whose last bits lie under bf16's least subnormal, 2^-133: the
+// sweep notes the least magnitude in each row and column (three more operations
+// a pair, in one of the two waves that split a fragment), and rows and columns
+// with such an element take their values from a second sweep on the fp32 MFMAs.
+// Before that check a product of operands near 1e-36 was off by 2.7e-5, near
+// 1e-38 by 2.7e-3 (now 1.4e-7); it costs 3 to 4% (4096^3 735 -> 759 us, 2048^3
+// 102.1 -> 105.7, 1000 x 1024 x 4096 59.6 -> 61.0).  Looking in both waves or by
+// v_cmp_class and scalar masks cost up to 10%, a second copy of the sweep with
+// the other fragments looked over 8%.
+// The product of two fragments is l h + h l + m m + m h + h m + h h on the bf16
+// matrix cores, summed in fp32, h h apart from the five small ones; the three
+// terms left out are below 2^-26 |x y|.  Six 32x32x16 bf16 MFMAs (192 cycles)
 // replace eight 32x32x2 fp32 ones (512 cycles).  What bounds it is the power
 // limit (the matrix pipes are 63% busy at 1.73 GHz) and the splitting's VALU
-// work, 44 operations per fragment, against 24 MFMAs per four fragments here;
+// work, 44 operations per fragment and 6 to look it over, against 24 MFMAs per
+// four fragments here;
 // on the 64 x 64 and 32 x 32 tiles, with one block per wave, the splitting
 // outweighs what the MFMAs save (784-256-256-10 at 64 rows 267 -> 297 us,
 // 1024-wide layers at 1024 rows 6.65 -> 6.75 ms), so those keep the fp32 MFMAs,
@@ -328,6 +338,13 @@ __device__ __forceinline__ void split3_pair(uint32_t x0, uint32_t x1, uint32_t& 
     const float t0 = r0 - __uint_as_float(m << 16), t1 = r1 - __uint_as_float(m & 0xFFFF0000u);
     l = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{t0, t1}, bf16x2));
 }
+// The least twice |x|'s bits less one (a zero's are all ones) of what was seen,
+// three operations a pair, and the value below which an element's pieces may be
+// short of it.
+__device__ __forceinline__ void split3_least(uint32_t& least, uint32_t x0, uint32_t x1) {
+    least = min(min(least, 2 * x0 - 1), 2 * x1 - 1);
+}
+constexpr uint32_t kSplit3Least = 2 * ((127u - 109u) << 23) - 1;
 
 // Workgroup ids are dealt round-robin over the XCDs (each with its own L2):
 // XCD x runs blocks x, x + 8, x + 16, ...
@@ -400,6 +417,18 @@ template <int W, int OPB> __device__ __forceinline__ int kn_row(int k) {
 template <int W, int OPB> __device__ __forceinline__ int kn_unit(int k, int unit) {
     if constexpr (OPB == 2) return unit ^ kn_swz<W>(k);
     else return W == 32 ? unit : unit ^ (((k >> 2) & 1) * 8);
+}
+// The 128 x 128 tile's: the offset of this lane's elements of chunk 0 at column
+// x, and the four from there on.  (32 columns on is a bit of the offset, 128.)
+template <int W> __device__ __forceinline__ uint32_t col_offset(int x) {
+    static_assert(W == 128, "the K row's bits lie above the unit's");
+    const int k = 4 * ((threadIdx.x & 63) >> 5);
+    return k * (W * 4) + kn_unit<W, 4>(k, x >> 2) * 16 + (x & 3) * 4;
+}
+__device__ __forceinline__ u32x4 col_read(const char* p) {
+    u32x4 v;
+    static_for<0, 4>([&](auto E) PCD_INLINE { v[decltype(E)::value] = *(const uint32_t*)(p + decltype(E)::value * 128 * 4); });
+    return v;
 }
 // This lane's four fp32 elements of chunk c (K rows 8c + 4 (lane / 32) ..+3)
 // at column x0 + lane % 32, from a region of K rows of W elements.
@@ -1282,8 +1311,11 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     };
     const int c0 = wk * C::NCW;   // this wave's first chunk of a stage
     bool op_mfmas = true;   // the sweep on the operand type's own MFMAs
-    // fp32 in bf16 pieces: the first sweep's elements where there is a second.
+    // fp32 in bf16 pieces: the first sweep's elements where there is a second, and
+    // which of them that one replaces (this lane's, and its registers' by bits).
     f32x16 first[SPLIT3 ? C::FM : 1][SPLIT3 ? C::FN : 1];
+    bool lane_lost[2];
+    uint32_t reg_lost[2];
     if constexpr (SPLIT3) {
         // Step kt (stage kt, 16 K elements of every row): the products of A's
         // first block row, then of its second.  One set of A's pieces is enough
@@ -1297,25 +1329,30 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         static_for<0, 4>([&](auto X) PCD_INLINE { small[decltype(X)::value / 2][decltype(X)::value % 2] = f32x16{}; });
         u32x4 ra[2][2], rb[2][2];   // fp32 elements of the fragments to split next
         Split3 pa[2], pb[2][2];
-        // Block row i of this wave's part of A, or block column i of B.
-        auto load_a = [&](int kt, int i, u32x4 (&raw)[2]) PCD_INLINE {
-            const char* st = smem + (kt % C::NS) * C::stage_bytes;
-            const int row = wm * C::WTM + i * 32 + lr;
+        // Block row i ^ wn of this wave's part of A, or block column j ^ wm of B:
+        // each fragment is split by the two waves that share it, and the one for
+        // which it is number 0 looks for elements that lose bits.  A lane's LDS
+        // address of a fragment's first chunk in stage 0; the second chunk of a
+        // row and the other block are a bit of it away.
+        const int ra0 = wm * C::WTM + wn * 32 + lr, rb0 = BM + wn * C::WTN + wm * 32 + lr;
+        const uint32_t at_a = AKM ? col_offset<BM>(ra0) : ra0 * C::RB + swz<C::RB>(ra0, half) * 16;
+        const uint32_t at_b = BKN ? BM * C::RB + col_offset<BN>(rb0 - BM) : rb0 * C::RB + swz<C::RB>(rb0, half) * 16;
+        constexpr uint32_t a_block = AKM ? 128 : 32 * C::RB, b_block = BKN ? 128 : 32 * C::RB;
+        static_assert(C::stage_bytes % (64 * C::RB) == 0 && BM * C::RB % (64 * C::RB) == 0, "the block's address bit");
+        auto load = [&](auto Cols, uint32_t at, u32x4 (&raw)[2]) PCD_INLINE {
             static_for<0, 2>([&](auto Cc) PCD_INLINE {
                 constexpr int c = decltype(Cc)::value;
-                if constexpr (AKM) raw[c] = col_fragment<BM>(st, c, wm * C::WTM + i * 32);
-                else raw[c] = *(const u32x4*)(st + row * C::RB + swz<C::RB>(row, 2 * c + half) * 16);
+                if constexpr (decltype(Cols)::value) raw[c] = col_read(smem + at + c * 8 * 128 * 4);
+                else raw[c] = *(const u32x4*)(smem + (at ^ (c * 32)));
             });
+        };
+        auto load_a = [&](int kt, int i, u32x4 (&raw)[2]) PCD_INLINE {
+            load(std::integral_constant<bool, AKM>{}, (kt % C::NS * C::stage_bytes + at_a) ^ (i * a_block), raw);
         };
         auto load_b = [&](int kt, int j, u32x4 (&raw)[2]) PCD_INLINE {
-            const char* st = smem + (kt % C::NS) * C::stage_bytes;
-            const int row = BM + wn * C::WTN + j * 32 + lr;
-            static_for<0, 2>([&](auto Cc) PCD_INLINE {
-                constexpr int c = decltype(Cc)::value;
-                if constexpr (BKN) raw[c] = col_fragment<BN>(st + BM * C::RB, c, wn * C::WTN + j * 32);
-                else raw[c] = *(const u32x4*)(st + row * C::RB + swz<C::RB>(row, 2 * c + half) * 16);
-            });
+            load(std::integral_constant<bool, BKN>{}, (kt % C::NS * C::stage_bytes + at_b) ^ (j * b_block), raw);
         };
+        uint32_t least_a = ~0u, least_b = ~0u;   // of the row of A's block 0, the column of B's that this lane holds part of
         auto split_half = [&](const u32x4& raw, Split3& d, auto E) PCD_INLINE {   // two pairs
             constexpr int e = decltype(E)::value;
             uint32_t h0, m0, l0, h1, m1, l1;
@@ -1330,6 +1367,10 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
             split_half(raw[0], d, std::integral_constant<int, 0>{});
             split_half(raw[1], d, std::integral_constant<int, 1>{});
         };
+        auto look = [&](const u32x4& raw, uint32_t& least) PCD_INLINE {
+            split3_least(least, raw[0], raw[1]);
+            split3_least(least, raw[2], raw[3]);
+        };
         auto piece = [](const Split3& p, int w) PCD_INLINE { return w == 0 ? p.h : w == 1 ? p.m : p.l; };
         // Product x (0..11) of block row i: term x / 2 (smallest first) of column x % 2.
         auto product = [&](auto I, auto Q, auto X) PCD_INLINE {
@@ -1340,18 +1381,27 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
             if constexpr (TRM) mfma_chunk<bf16_t>(to, bv, av);
             else mfma_chunk<bf16_t>(to, av, bv);
         };
-        // Block row i's 12 products with the splitting of two fragments, a quarter of it after every third.
-        auto half_step = [&](auto I, auto Q, const u32x4 (&r0)[2], Split3& d0, const u32x4 (&r1)[2], Split3& d1) PCD_INLINE {
+        // Block row i's 12 products with the splitting of two fragments, a quarter of it after every third;
+        // fragment F of the two, a block 0, is looked over, unless it is past the last stage (not `live`).
+        auto half_step = [&](auto I, auto Q, const u32x4 (&r0)[2], Split3& d0, const u32x4 (&r1)[2], Split3& d1, auto F,
+                             uint32_t& least, bool live) PCD_INLINE {
+            uint32_t seen = least;
             static_for<0, 4>([&](auto G) PCD_INLINE {
                 constexpr int g = decltype(G)::value;
+                constexpr bool looks = g / 2 == decltype(F)::value;
                 static_for<3 * g, 3 * g + 3>([&](auto X) PCD_INLINE { product(I, Q, X); });
                 split_half(g < 2 ? r0[g % 2] : r1[g % 2], g < 2 ? d0 : d1, std::integral_constant<int, g % 2>{});
+                if constexpr (looks) {
+                    look(g < 2 ? r0[g % 2] : r1[g % 2], seen);
+                    asm volatile("" : "+v"(seen));   // here, not behind a branch on `live`
+                }
                 static_for<0, 3>([&](auto) PCD_INLINE {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, looks ? 10 : 8, 0);
                 });
                 __builtin_amdgcn_sched_barrier(0);
             });
+            least = live ? seen : least;
         };
         // Like stage_ready, with one stage less in flight: a stage's slot is
         // refilled after the barrier that follows its last read.
@@ -1367,16 +1417,17 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         const std::integral_constant<int, 1> I1{};
         auto step = [&](auto Q, int kt) PCD_INLINE {
             constexpr int q = decltype(Q)::value;
+            const bool live = kt + 1 < nk;
             load_a(kt + 1, 0, ra[0]);
             load_b(kt + 1, 1, rb[1]);
             __builtin_amdgcn_sched_barrier(0);
-            half_step(I0, Q, ra[1], pa[1], rb[0], pb[q ^ 1][0]);
+            half_step(I0, Q, ra[1], pa[1], rb[0], pb[q ^ 1][0], I1, least_b, live);
             if (kt + 2 < nk) ready(kt + 2);
             if (kt + 1 + C::D < nk) issue_stage(kt + 1 + C::D);
             load_a(kt + 1, 1, ra[1]);
             load_b(kt + 2, 0, rb[0]);
             __builtin_amdgcn_sched_barrier(0);
-            half_step(I1, Q, ra[0], pa[0], rb[1], pb[q ^ 1][1]);
+            half_step(I1, Q, ra[0], pa[0], rb[1], pb[q ^ 1][1], I0, least_a, live);
         };
         // Past the last stage the reads and splits run on whatever the ring holds, unused.
         for (int s2 = 0; s2 < C::D && s2 < nk; ++s2) issue_stage(s2);
@@ -1388,6 +1439,10 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         split_frag(ra[0], pa[0]);
         split_frag(rb[0], pb[0][0]);
         split_frag(rb[1], pb[0][1]);
+        static_for<0, 2>([&](auto Cc) PCD_INLINE {
+            look(ra[0][decltype(Cc)::value], least_a);
+            look(rb[0][decltype(Cc)::value], least_b);
+        });
         if (nk > 1) ready(1);
         if (C::D < nk) issue_stage(C::D);
         load_b(1, 0, rb[0]);
@@ -1398,34 +1453,52 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
         }
         if (kt < nk) step(I0, kt);
         static_for<0, 4>([&](auto X) PCD_INLINE { accs[0][decltype(X)::value / 2][decltype(X)::value % 2] += small[decltype(X)::value / 2][decltype(X)::value % 2]; });
-        // An element that is not finite: an operand was not (its pieces mix
-        // infinities and NaNs), it rounded up to infinity as a bf16, or the sum
-        // overflowed.  Such elements take the values of a second sweep, on the
-        // fp32 MFMAs, which give their own infinities and NaNs; the tile's other
-        // elements keep theirs, so what a row gets does not depend on the rows
-        // beside it.  Rows that are not stored do not ask for that sweep (a
+        auto exchange = [](f32x16& a, f32x16& b) PCD_INLINE { const f32x16 t = a; a = b; b = t; };
+        if (wave_u % C::WN) exchange(accs[0][0][0], accs[0][1][0]), exchange(accs[0][0][1], accs[0][1][1]);   // to their places
+        if (wave_u / C::WN) exchange(accs[0][0][0], accs[0][0][1]), exchange(accs[0][1][0], accs[0][1][1]);
+        // Elements that the pieces do not give as the fp32 MFMAs do: one that is
+        // not finite (an operand was not, and its pieces mix infinities and
+        // NaNs; it rounded up to infinity as a bf16; or the sum overflowed), and
+        // every element of a row or column with an operand that loses bits.
+        // Those take the values of a second sweep, on the fp32 MFMAs; the tile's
+        // other elements keep theirs, so what a row gets does not depend on the
+        // rows beside it.  Rows that are not stored do not ask for that sweep (a
         // settling's rows past M hold what earlier calls left there, and a
         // ragged settling's rows that have left keep their states).
+        typedef volatile __attribute__((address_space(3))) uint32_t lds_u32;
+        lds_u32* word = (lds_u32*)smem;   // the flag, then A's rows and B's columns, 32 to a word
+        __syncthreads();                  // every wave is done reading the stage ring
+        const uint64_t lost_a = __ballot(least_a < kSplit3Least), lost_b = __ballot(least_b < kSplit3Least);
+        if (lane == 0) {
+            word[1 + wm * 2 + wn] = (uint32_t)(lost_a | lost_a >> 32);
+            word[5 + wn * 2 + wm] = (uint32_t)(lost_b | lost_b >> 32);
+        }
+        if (tid == 0) word[0] = 0;
+        __syncthreads();
+        static_for<0, 2>([&](auto X) PCD_INLINE {
+            constexpr int x = decltype(X)::value;
+            const uint32_t a = word[1 + wm * 2 + x], b = word[5 + wn * 2 + x];
+            lane_lost[x] = (TRM ? a : b) >> lr & 1;
+            reg_lost[x] = (TRM ? b : a) >> 4 * half;
+        });
         bool again = false;
         static_for<0, C::FM>([&](auto I) PCD_INLINE {
             constexpr int i = decltype(I)::value;
             bool bad = false;
             static_for<0, C::FN>([&](auto J) PCD_INLINE {
+                constexpr int j = decltype(J)::value;
+                bad |= lane_lost[TRM ? i : j] || reg_lost[TRM ? j : i] != 0;
                 static_for<0, 16>([&](auto R) PCD_INLINE {
-                    bad |= !(fabsf(accs[0][i][decltype(J)::value][decltype(R)::value]) <= 3.402823466e38f);
+                    bad |= !(fabsf(accs[0][i][j][decltype(R)::value]) <= 3.402823466e38f);
                 });
             });
             const int row = row0 + wm * C::WTM + i * 32 + lr;
             if (TRM && bad) bad = row < P.M && row_active(args, row);
             again |= bad;
         });
-        volatile __attribute__((address_space(3))) int* flag = (volatile __attribute__((address_space(3))) int*)smem;
-        __syncthreads();   // every wave is done reading the stage ring
-        if (tid == 0) *flag = 0;
+        if (again) word[0] = 1;
         __syncthreads();
-        if (again) *flag = 1;
-        __syncthreads();
-        op_mfmas = *flag != 0;
+        op_mfmas = word[0] != 0;
         if (op_mfmas) {
             __syncthreads();
             static_for<0, C::FM>([&](auto I) PCD_INLINE {
@@ -1478,7 +1551,9 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
                     static_for<0, 16>([&](auto R) PCD_INLINE {
                         constexpr int i = decltype(I)::value, j = decltype(J)::value, r = decltype(R)::value;
                         const float v = first[i][j][r];
-                        if (fabsf(v) <= 3.402823466e38f) accs[0][i][j][r] = v;
+                        const bool replaced = !(fabsf(v) <= 3.402823466e38f) || lane_lost[TRM ? i : j] ||
+                                              (reg_lost[TRM ? j : i] >> (8 * (r >> 2) + (r & 3)) & 1);
+                        if (!replaced) accs[0][i][j][r] = v;
                     });
                 });
             });

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from predicitivecoding_amd import PcDeviceModel
+from predicitivecoding_amd import GenerativeSnapshot, PcDeviceModel
 from predicitivecoding_amd._native import call
 from tests.test_gpu_shared_rows import network, settle
 
@@ -101,3 +101,65 @@ def test_ragged_order_does_not_matter():
     for a, b in zip(*out):
         np.testing.assert_array_equal(np.asarray(a), np.asarray(b))
     model.close()
+
+
+# magnitudes from where three bf16 pieces hold every fp32 bit to the smallest subnormals; in every layout, as the
+# operand's fragments come out of LDS in two ways
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 1), (1, 0)])
+@pytest.mark.parametrize("scale", [1e-32, 1e-33, 1e-34, 1e-36, 1e-38, 1e-41])
+def test_small_operands_keep_their_bits(ta, tb, scale):
+    """An operand whose third bf16 piece would be below bf16's range takes the fp32 MFMAs, in rows and in columns: one
+    rounding (2^-24 / sqrt(3) in the mean square) per two of K = 64 elements, twice that."""
+    A, B = operands(64, 9)
+    A[:700] *= scale
+    A[700:] *= 1e25
+    A[1500, 63] = scale
+    B[1900:] *= scale
+    C, ref = product(A, B, ta, tb), A.double() @ B.double().T
+    bound = 2 * 2.0 ** -24 / np.sqrt(3.0) * np.sqrt(64 / 2 + 1)
+    parts = [(slice(700, 2048), slice(1900, 2048)), (slice(700, 2048), slice(0, 1900)), (1500, slice(0, 2048))]
+    if scale > 1e-37:   # the products themselves in the normal range
+        parts.append((slice(0, 700), slice(0, 1900)))
+    for r, c in parts:
+        err = (C[r, c].double() - ref[r, c]).norm() / ref[r, c].norm()
+        assert float(err) <= bound, (r, c, float(err), bound)
+
+
+@pytest.mark.parametrize("which", ["row", "column"])
+@pytest.mark.parametrize("k", [0, 15, 16, 33, 207])
+def test_one_small_operand_is_found_wherever_it_lies(which, k):
+    """A single product is one rounding from exact; its neighbours keep their bits.  K elements of the first, middle and
+    last stages; rows and columns of each of the waves' blocks."""
+    A, B = operands(208, 3)
+    C0 = product(A, B)
+    at = torch.tensor([1, 33, 65, 97, 128 + 50, 2047], device="cuda")
+    v = torch.full((6,), 1.2345678e-36, device="cuda")
+    X, Y = (A, B) if which == "row" else (B, A)
+    X[at] = 0.0
+    X[at, k] = v
+    Y[300, k] = 3.1415926e30
+    C = product(A, B)
+    got = C[at, 300] if which == "row" else C[300, at]
+    want = v.double() * Y[300, k].double()
+    assert float(((got.double() - want) / want).abs().max()) <= 2.0 ** -24
+    keep = torch.ones(2048, dtype=torch.bool, device="cuda")
+    keep[at] = False
+    other = torch.ones(2048, dtype=torch.bool, device="cuda")
+    other[300] = False
+    a, b = (keep, other) if which == "row" else (other, keep)
+    assert torch.equal(C[a][:, b], C0[a][:, b])
+
+
+def test_small_states_settle_as_on_the_64_tile():
+    """A linear network without biases scales: inputs of 2^-121 give the settling of unit inputs, scaled, where the
+    64 x 64 tile's fp32 MFMAs do."""
+    net = GenerativeSnapshot(SIZES, 0, 0.1, 0.0, False, network(SIZES, 0).weights,
+                             [np.zeros(n, np.float32) for n in SIZES[:-1]])
+    x = torch.randn(300, SIZES[0], generator=torch.Generator().manual_seed(4)).cuda()
+    model = PcDeviceModel(net, "f32")
+    model.set_option("tile", 128)
+    unit = settle(model, x, 5)[0].astype(np.float64)
+    small = settle(model, x * 2.0 ** -121, 5)[0].astype(np.float64) * 2.0 ** 121
+    model.close()
+    # fp32 roundings of 5 steps, and of states near 2^-126 to multiples of 2^-149: 2^-23 of them
+    assert np.linalg.norm(small - unit) / np.linalg.norm(unit) <= 2e-6
