@@ -306,8 +306,10 @@ template <> __device__ __forceinline__ void mfma_chunk<f16_t>(f32x16& acc, const
 // v_cmp_class and scalar masks cost up to 10%, a second copy of the sweep with
 // the other fragments looked over 8%.
 // The product of two fragments is l h + h l + m m + m h + h m + h h on the bf16
-// matrix cores, summed in fp32, h h apart from the five small ones; the three
-// terms left out are below 2^-26 |x y|.  Six 32x32x16 bf16 MFMAs (192 cycles)
+// matrix cores, summed in fp32, h h apart from the five small ones.  The three
+// terms left out are below 2^-24 |x y| (|m| reaches 2^-8 |x| and |l| 2^-17 |x|),
+// at most what rounding that product to fp32 would cost, and 2^-27 of it in the
+// root mean square over normal operands.  Six 32x32x16 bf16 MFMAs (192 cycles)
 // replace eight 32x32x2 fp32 ones (512 cycles).  What bounds it is the power
 // limit (the matrix pipes are 63% busy at 1.73 GHz) and the splitting's VALU
 // work, 44 operations per fragment and 6 to look it over, against 24 MFMAs per

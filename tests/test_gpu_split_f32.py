@@ -33,7 +33,8 @@ def test_split_products_against_64_bits(m, n, k, scale):
     ref = A.double() @ B.double().T
     err = (product(A, B).double() - ref).norm() / ref.norm()
     # One rounding (2^-24 / sqrt(3) of the value in the mean square) per 16 elements of K of a sum that grows to its
-    # final size, one when the small products join it, twice that; and the terms left out (2^-26).
+    # final size, one when the small products join it, twice that; and the terms left out
+    # (2^-27 of normal operands' products in the root mean square, 2^-24 at most), twice that.
     bound = 2 * 2.0 ** -24 / np.sqrt(3.0) * np.sqrt(np.ceil(k / 16.0) + 1) + 2.0 ** -26
     assert float(err) <= bound, (float(err), bound)
 
@@ -54,3 +55,17 @@ def test_special_operands_as_fp32_multiplies_them(special):
     assert torch.equal(torch.isinf(C) & (C < 0), torch.isinf(ref32) & (ref32 < 0))
     ok = torch.isfinite(ref32) & (ref.abs() < 1e6)
     assert float((C.double() - ref)[ok].abs().max()) < 1e-4   # K = 256 unit normals: 5e-6 at most
+
+
+@pytest.mark.parametrize("k", [16, 64, 208, 1024])
+def test_operands_that_lose_most(k):
+    """The products left out are largest, and all of one sign, where both operands are 1 + 2^-8 - 2^-17 times a power of
+    two: 2^-24 of each product.  Beside that, at most one rounding (2^-24) of a growing sum per 16 elements of K, one
+    of the small products' sum and one when it joins."""
+    v = 1 + 2.0 ** -8 - 2.0 ** -17
+    g = torch.Generator(device="cuda").manual_seed(k)
+    e = torch.randint(-6, 7, (2, 2048, k), generator=g, device="cuda", dtype=torch.float32)
+    A, B = v * torch.exp2(e[0]), v * torch.exp2(e[1])
+    ref = A.double() @ B.double().T
+    err = float(((product(A, B).double() - ref) / ref).abs().max())
+    assert err <= 2.0 ** -24 * (1 + k / 16 + 2), err
