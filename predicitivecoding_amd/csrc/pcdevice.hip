@@ -1678,10 +1678,11 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     a.item_b = (size_t)n * kp * ob;
     a.item_c = (size_t)m * n;
     const int epi = mk_a ? (kn_b ? EPI_PLAIN_MKKN : EPI_PLAIN_MK) : (kn_b ? EPI_PLAIN_KN : EPI_PLAIN);
-    // Launches of at most 2^24 work units (one, but for batches of millions).
-    const int most = std::max(1, (1 << 24) / a.item_tiles);
-    for (int i0 = 0; i0 < batch && !st; i0 += most) {
-        a.items = std::min(most, batch - i0);
+    // Launches of at most 2^22 work units (one, but for batches of millions):
+    // HIP takes fewer than 2^32 threads in a grid, and a unit has up to 512.
+    const int most = std::max(1, (1 << 22) / a.item_tiles);
+    for (long i0 = 0; i0 < batch && !st; i0 += most) {
+        a.items = (int)std::min<long>(most, batch - i0);
         if (batch > 1) p.tiles = a.items * a.item_tiles;
         st = launch_phase(dtype, tile, epi, sets[0], a, s);
         p.A = (const char*)p.A + most * a.item_a;
