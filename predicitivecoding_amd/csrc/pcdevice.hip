@@ -1572,7 +1572,7 @@ static Tile choose_gemm_tile(int dtype, int m, int k, int n, int cus, int batch 
 // Gemm.MatMul's own row-major [k x n] layout and a transposed A ([k x m]) through
 // EPI_PLAIN_KN, _MK and _MKKN, which take K rows of the tile's columns.  Rows
 // and columns need no whole tiles (the kernel repeats the last ones).  Any
-// other operand is packed K-contiguous, K padded with zeros, into scratch.
+// other operand, and one that the result lies over, is packed K-contiguous, K padded with zeros, into scratch.
 // All products run in one launch (their tiles dealt over the XCDs together).
 // Measured, packing whatever filled no whole tiles -> in place: 1000 x 1024 x
 // 4096 fp32 row-major 69 -> 62 us; 1000 x 4096 x 4096 bf16 57 -> 50 us; 96 x
@@ -1589,8 +1589,10 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     const Tile tile = choose_gemm_tile(dtype, m, k, n, cus, batch);
     const int ob = op_bytes(dtype), unit = 16 / ob;
     const int kp = (int)round_up(k, stage_k(dtype, tile));
-    auto aligned = [&](const void* p, size_t item) {
-        return (uintptr_t)p % 16 == 0 && (batch == 1 || item * ob % 16 == 0);
+    const uintptr_t c0 = (uintptr_t)dC, c1 = c0 + (size_t)batch * m * n * 4;
+    auto in_place = [&](const void* p, size_t item) {
+        const uintptr_t p0 = (uintptr_t)p, p1 = p0 + (size_t)batch * item * ob;
+        return p0 % 16 == 0 && (batch == 1 || item * ob % 16 == 0) && (p1 <= c0 || c1 <= p0);
     };
     // Except that the transposing reads cost the 16-bit 128 x 128 tile about a
     // fifth of its time, more than packing an operand a quarter the other's size
@@ -1599,10 +1601,10 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     const bool small_a = ob == 2 && tile.m == 128 && (size_t)m * 4 <= (size_t)n;
     const bool small_b = ob == 2 && tile.m == 128 && (size_t)n * 4 <= (size_t)m;
     const bool whole_k = k == kp, kn = whole_k && kn_tile(ob, tile.m, tile.n, false);
-    const bool direct_a = whole_k && !trans_a && k % unit == 0 && aligned(dA, (size_t)m * k);
-    const bool direct_b = whole_k && trans_b && k % unit == 0 && aligned(dB, (size_t)k * n);
-    const bool mk_a = kn && trans_a && !small_a && m % unit == 0 && aligned(dA, (size_t)m * k);
-    const bool kn_b = kn && !trans_b && !small_b && n % unit == 0 && aligned(dB, (size_t)k * n);
+    const bool direct_a = whole_k && !trans_a && k % unit == 0 && in_place(dA, (size_t)m * k);
+    const bool direct_b = whole_k && trans_b && k % unit == 0 && in_place(dB, (size_t)k * n);
+    const bool mk_a = kn && trans_a && !small_a && m % unit == 0 && in_place(dA, (size_t)m * k);
+    const bool kn_b = kn && !trans_b && !small_b && n % unit == 0 && in_place(dB, (size_t)k * n);
     void *pa = nullptr, *pb = nullptr, *part = nullptr;
     auto pack = [&](const void* src, int rows, int trans, void* dst) -> int {
         const int f32 = dtype == PCD_F32;
