@@ -52,6 +52,7 @@ sys.path.insert(0, ROOT)
 
 PEAK = {"f32": 157.3e12, "bf16": 2.5e15, "f16": 2.5e15}   # dense MFMA, MI355X
 HBM_PEAK = 8.0e12
+CUS = 256
 
 CONFIGS = {
     "c1": dict(sizes=[784, 256, 256, 10], act=1, dtype="f32", batch=64, T=20, eta=0.1, x="uniform01", init="xavier"),
@@ -100,8 +101,24 @@ def apply_options(model, args):
         model.set_option(name, int(value))
 
 
-def flops_per_sample_step(sizes):
-    return 4.0 * sum(sizes[l] * sizes[l - 1] for l in range(1, len(sizes)))
+def mfma_peak(sizes, rows, dtype, tile=0):
+    """The MFMA rate that bounds a settling's products.  fp32 on the library's
+    128 x 128 tile multiplies three bf16 pieces of each operand, six products
+    for one, so a sixth of the bf16 rate bounds it; the other tiles are bound by
+    the fp32 MFMAs.  The workloads here take that tile where their error phase
+    has one for every CU."""
+    tiles = -(-rows // 128) * sum(-(-s // 128) for s in sizes[:-1])
+    if dtype == "f32" and (tile == 128 or (tile == 0 and tiles >= CUS)):
+        return PEAK["bf16"] / 6
+    return PEAK[dtype]
+
+
+def path_flops(sizes, B, T, shared_rows):
+    """FLOPs of one fixed-step settling.  Layers the input has not reached are
+    settled as one row (not counted) where `shared_rows`: layer l's two problems
+    are then the batch's in steps l - 1 .. T - 1, otherwise in all T."""
+    return 4.0 * B * sum(sizes[l] * sizes[l - 1] * (max(0, T - l + 1) if shared_rows else T)
+                         for l in range(1, len(sizes)))
 
 
 def phase_bytes(sizes, B, dtype):
@@ -416,7 +433,7 @@ def bench_ragged(args, cfg):
     flop_launch = 2.0 * S * active.mean()             # mean over the launches of one phase
     dom_name, dom_ms = ("update_phase", upd_ms) if upd_ms >= err_ms else ("error_phase", err_ms)
     achieved = flop_launch / (dom_ms * 1e-3)
-    peak = PEAK[cfg["dtype"]]
+    peak = mfma_peak(sizes, rows, cfg["dtype"], args.tile)
     roofline = {"bound": "mfma", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                 "frac": achieved / peak, "traffic": traffic_from_profiles(args.config, dom_name), "kernel": dom_name,
                 "kernel_ms": dom_ms, "error_phase_ms": err_ms, "update_phase_ms": upd_ms, "launches_timed": launches,
@@ -503,7 +520,7 @@ def bench_clamped(args, cfg):
     ms = {"error_phase": err_ms, "update_phase": upd_ms}
     dom_name = max(ms, key=ms.get)
     achieved = flops[dom_name] / (ms[dom_name] * 1e-3)
-    peak = PEAK[cfg["dtype"]]
+    peak = mfma_peak(sizes, rows, cfg["dtype"], args.tile)
     roofline = {"bound": "mfma", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                 "frac": achieved / peak, "traffic": traffic_from_profiles(args.config, dom_name), "kernel": dom_name,
                 "kernel_ms": ms[dom_name], "error_phase_ms": err_ms, "update_phase_ms": upd_ms,
@@ -855,7 +872,8 @@ def bench_settle(args, name, cfg, steps, warmup, cpu_budget, pcie=False):
     model.set_option("profile", 1)
     err_ms = upd_ms = 0.0
     launches = 0
-    for _ in range(max(1, min(steps, 5))):
+    profiled = max(1, min(steps, 5))
+    for _ in range(profiled):
         one_pass()
         e, u, n = model.profile_result()
         err_ms += e * n
@@ -869,7 +887,9 @@ def bench_settle(args, name, cfg, steps, warmup, cpu_budget, pcie=False):
     flop_launch = 2.0 * B * sum(sizes[l] * sizes[l - 1] for l in range(1, len(sizes)))
     bytes_err, bytes_upd = phase_bytes(sizes, B, cfg["dtype"])
     bytes_launch = bytes_upd if dom_name == "update_phase" else bytes_err
-    peak = PEAK[cfg["dtype"]]
+    peak = mfma_peak(sizes, B, cfg["dtype"], args.tile)
+    # (steps with one-row layers are not timed: there are fewer timed launches than steps)
+    flop_pass = path_flops(sizes, B, T, shared_rows=launches < profiled * T)
     # The roofline the arithmetic names: HBM when the launch's FLOP per
     # algorithmic byte is below the ridge (peak FLOP/s / peak HBM bytes/s).
     if flop_launch / bytes_launch < peak / HBM_PEAK:
@@ -888,7 +908,7 @@ def bench_settle(args, name, cfg, steps, warmup, cpu_budget, pcie=False):
                     "frac": achieved / peak, "traffic": traffic_from_profiles(name, dom_name),
                     "kernel": dom_name, "kernel_ms": dom_ms, "error_phase_ms": err_ms, "update_phase_ms": upd_ms,
                     "flop_per_launch": flop_launch, "bytes_per_launch": bytes_launch, "launches_timed": launches,
-                    "path_frac": (flops_per_sample_step(sizes) * value) / peak,
+                    "flop_per_pass": flop_pass, "path_frac": flop_pass / (ms_per_step * 1e-3) / peak,
                     # the same launch against the HBM roofline: algorithmic bytes / duration
                     "hbm_achieved_GBps": bytes_launch / (dom_ms * 1e-3) / 1e9,
                     "hbm_frac": bytes_launch / (dom_ms * 1e-3) / HBM_PEAK}
