@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ src0
         for (int by = blockIdx.y; by < tiles_y; by += gridDim.y) {
             const int r0 = by * 64;
             const int sr0 = trans ? c0 : r0, sc0 = trans ? r0 : c0;   // the tile's origin in the physical source
-    #pragma unroll
+#pragma unroll
             for (int i = qr; i < 64; i += 16) {
                 const int sr = sr0 + i, sc = sc0 + q4;
                 uint32_t w[4] = {0u, 0u, 0u, 0u};
@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ src0
                 }
             }
             __syncthreads();
-    #pragma unroll
+#pragma unroll
             for (int i = qr; i < 64; i += 16) {
                 const int r = r0 + i, c = c0 + q4;
                 if (r >= prow || c >= pcol) continue;
@@ -177,7 +177,7 @@ __global__ void exit_kernel(const float* __restrict__ part, int ldp, int nslots,
     const int r0 = row_offsets[r], r1 = row_offsets[r + 1];
     float s = 0.f;
     for (int row = r0 + threadIdx.x; row < r1; row += blockDim.x)
-        s += sum_slots(part, ldp, nslots, row, nslots);
+        s += sum_slots(part, ldp, nslots, row);
     __shared__ float red[256];
     red[threadIdx.x] = s;
     __syncthreads();
@@ -205,7 +205,7 @@ __global__ void exit_rows_kernel(const float* __restrict__ part, int ldp, int ns
                                  float* __restrict__ last_energy, int t, int rule, float thr) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < requests; r += gridDim.x * blockDim.x) {
         if (t >= done_at[r]) continue;
-        const float e = sum_slots(part, ldp, nslots, r, nslots);
+        const float e = sum_slots(part, ldp, nslots, r);
         const float prev = prev_energy[r];
         bool stop = false;
         if (rule == 1) stop = thr > 0.f && t > 0 && (prev - e < thr * fmaxf(prev, 1e-12f));
@@ -307,7 +307,7 @@ active_tiles_kernel(const int* __restrict__ row_offsets, const int* __restrict__
 __global__ void energy_rows_kernel(const float* __restrict__ part, int ldp, int nslots, float* __restrict__ out,
                                    int rows) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
-        out[r] = sum_slots(part, ldp, nslots, r, nslots);
+        out[r] = sum_slots(part, ldp, nslots, r);
     }
 }
 

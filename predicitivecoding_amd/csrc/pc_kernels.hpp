@@ -113,9 +113,20 @@ struct Problem {
     int tiles_m, tiles_n;  // tile grid of the output
     int tiles;            // work units: tiles_m * tiles_n * ksplit
     int ldo;              // leading dimension of every [rows x N] epilogue operand
-    const float* bias;    // ERROR/FFG: b_l [N]
-    const float* mlow;    // ERROR: fp32 state M_{l-1}; UPDATE: fp32 state M_l before the step (read at the top layer)
-    float* eout;          // ERROR: X_{l-1} = M - eta (E + lambda sign M) (nullable: layer 0 is never updated)
+    // PLAIN: `tiles` may be those of several products of this shape; item_a, item_b bytes of A, B and item_c elements
+    // of C from one to the next.  (Not in PhaseArgs: the settling kernels' arguments stay as short as they can be.)
+    union {
+        const float* bias;    // ERROR/FFG: b_l [N]
+        size_t item_a;
+    };
+    union {
+        const float* mlow;    // ERROR: fp32 state M_{l-1}; UPDATE: fp32 state M_l before the step (read at the top layer)
+        size_t item_b;
+    };
+    union {
+        float* eout;          // ERROR: X_{l-1} = M - eta (E + lambda sign M) (nullable: layer 0 is never updated)
+        size_t item_c;
+    };
     void* dout;           // ERROR: D_l in the operand type; FFG: operand-type state copy
     float* m;             // UPDATE: fp32 state M_l out; FFG: state out; PLAIN: C
     void* mop;            // UPDATE: operand-type copy of M_l (nullable for fp32)
@@ -168,9 +179,12 @@ struct PhaseArgs {
     const int* act_count;       // ragged: their number
     int nt_store;               // settling epilogues store their full rows non-temporally
     int nt_load;                // settling epilogues load their fp32 state rows non-temporally
-    int items, item_tiles;      // PLAIN: products of the launch's one shape (<= 1: one) and the work units of each
-    size_t item_a, item_b, item_c;   // PLAIN: bytes from one product's A, B to the next, elements of its C
 };
+// A small settling's launches read their arguments first, from memory: four
+// words of these more, and a longer prologue of the energies' sum, made
+// settlings on the 32 x 32 tile 0.3 to 1% slower (10 x 456 f16 at 5 rows 304 ->
+// 307 us, 784-256-256-10 fp32 at 64 258.1 -> 258.9).
+static_assert(sizeof(PhaseArgs) <= 104, "the settling kernels' arguments");
 
 // How a phase's tiles are dealt over the XCDs.
 enum TileOrder { TILE_INTERLEAVED = 0, TILE_CONTIGUOUS = 1 };
@@ -359,11 +373,24 @@ __host__ __device__ __forceinline__ void xcd_share(int n, int x, int& lo, int& c
     cnt = n * (x + 1) / kXcds - lo;
 }
 
-// Sum of a row's energy partials over the slots, in slot order (slots from
-// shared_from on are row 0's for every row).  The loads go out eight at a time
-// ahead of the adds (one dependent load per slot would pay the memory latency
-// nslots times).
-__device__ __forceinline__ float sum_slots(const float* part, int ldp, int nslots, int row, int shared_from) {
+// Sum of a row's energy partials over the slots, in slot order.  The loads
+// go out eight at a time ahead of the adds (one dependent load per slot would
+// pay the memory latency nslots times).
+__device__ __forceinline__ float sum_slots(const float* part, int ldp, int nslots, int row) {
+    float s = 0.f;
+    int k = 0;
+    for (; k + 8 <= nslots; k += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = gld(part + (size_t)(k + j) * ldp + row);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += v[j];
+    }
+    for (; k < nslots; ++k) s += gld(part + (size_t)k * ldp + row);
+    return s;
+}
+// The same where the slots from shared_from on hold row 0's for every row.
+__device__ __forceinline__ float sum_shared_slots(const float* part, int ldp, int nslots, int row, int shared_from) {
     float s = 0.f;
     int k = 0;
     auto add = [&](const float* at, int end) PCD_INLINE {
@@ -947,9 +974,12 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // whose phases are latency-bound, then starts without this delay.
     if (EPI == EPI_UPDATE && args.energy_out != nullptr) {
         for (int row = (vgrid - 1 - vblock) * C::NT + tid; row < args.batch; row += vgrid * C::NT) {
-            gst(args.energy_out + (size_t)args.t * args.batch + row,
-                sum_slots(args.energy_part, args.ldp, args.nslots, row,
-                          C::KSW || C::WD ? args.nslots : args.shared_from));   // (no one-row layers on those tiles)
+            float e;
+            if constexpr (C::KSW || C::WD)   // no one-row layers on those tiles
+                e = sum_slots(args.energy_part, args.ldp, args.nslots, row);
+            else
+                e = sum_shared_slots(args.energy_part, args.ldp, args.nslots, row, args.shared_from);
+            gst(args.energy_out + (size_t)args.t * args.batch + row, e);
         }
     }
 
@@ -999,12 +1029,13 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     if (local < 0) return;  // a spare workgroup of this XCD (the grid is 8 x the largest XCD share)
     Problem P = load_problem(kprobs + p);
     if constexpr (EPI >= EPI_PLAIN) {
-        if (args.items > 1) {   // one of several products of the same shape
-            const int item = local / args.item_tiles;
-            local -= item * args.item_tiles;
-            P.A = (const char*)P.A + item * args.item_a;
-            P.B = (const char*)P.B + item * args.item_b;
-            P.m += item * args.item_c;
+        const int item_tiles = P.tiles_m * P.tiles_n * max(P.ksplit, 1);
+        if (P.tiles > item_tiles) {   // several products of the same shape
+            const int item = local / item_tiles;
+            local -= item * item_tiles;
+            P.A = (const char*)P.A + item * P.item_a;
+            P.B = (const char*)P.B + item * P.item_b;
+            P.m += item * P.item_c;
         }
     }
     // Split-K: unit `local` is K range `split` of tile `local / ksplit` (a

@@ -1675,21 +1675,19 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     a.beta = beta;
     a.k_stagger = dtype == PCD_F32 ? 0 : auto_k_stagger(kp / stage_k(dtype, tile));
     a.nt_store = (size_t)batch * m * n * 4 >= kGemmNtBytes;
-    a.item_tiles = p.tiles_m * p.tiles_n;
-    a.item_a = (size_t)m * kp * ob;
-    a.item_b = (size_t)n * kp * ob;
-    a.item_c = (size_t)m * n;
+    p.item_a = (size_t)m * kp * ob;
+    p.item_b = (size_t)n * kp * ob;
+    p.item_c = (size_t)m * n;
     const int epi = mk_a ? (kn_b ? EPI_PLAIN_MKKN : EPI_PLAIN_MK) : (kn_b ? EPI_PLAIN_KN : EPI_PLAIN);
     // Launches of at most 2^22 work units (one, but for batches of millions):
     // HIP takes fewer than 2^32 threads in a grid, and a unit has up to 512.
-    const int most = std::max(1, (1 << 22) / a.item_tiles);
+    const int item_tiles = p.tiles_m * p.tiles_n, most = std::max(1, (1 << 22) / item_tiles);
     for (long i0 = 0; i0 < batch && !st; i0 += most) {
-        a.items = (int)std::min<long>(most, batch - i0);
-        if (batch > 1) p.tiles = a.items * a.item_tiles;
+        if (batch > 1) p.tiles = (int)std::min<long>(most, batch - i0) * item_tiles;
         st = launch_phase(dtype, tile, epi, sets[0], a, s);
-        p.A = (const char*)p.A + most * a.item_a;
-        p.B = (const char*)p.B + most * a.item_b;
-        p.m += most * a.item_c;
+        p.A = (const char*)p.A + most * p.item_a;
+        p.B = (const char*)p.B + most * p.item_b;
+        p.m += most * p.item_c;
     }
     for (void* q : {pa, pb, part})
         if (q) {
