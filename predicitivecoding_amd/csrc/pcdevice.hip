@@ -570,18 +570,34 @@ int max_energy_slots(const pcd_model* m) {
     return slots;
 }
 
-// Launches pack_kernel over the [prow x pcol] destination: 64 x 64 tiles, a
+// Packs `items` matrices into [prow x pcol] destinations.  64 x 64 tiles, a
 // column of tiles per workgroup column, about 4096 workgroups in all (each
-// walks down several tile rows when the matrix is large).
+// walks down several tile rows when the matrix is large); up to 2^19 elements,
+// where the tiles' way through LDS takes longer than it saves, a thread per
+// element (2 x (225 x 195 x 448) fp32 products, 220000 and fewer elements per
+// operand, 14.0 with tiles, 11.1 with elements; 40 x (100 x 101 x 52), 450000,
+// 15.4 and 13.4; 1000 x 1001 x 1000, a million, 37.0 and 37.8; 96 x (200 x 65 x
+// 200), 1.5 million, 33.0 and 35.2).
+constexpr size_t kPackSmall = (size_t)1 << 19;
 template <typename OP>
 void pack_op(hipStream_t s, const void* src, int src_is_f32, int rows, int cols, int trans, void* dst, int prow,
              int pcol, int ldd, int items = 1) {
+    const size_t n = (size_t)items * prow * pcol;
+    if (ldd == pcol && n <= kPackSmall) {
+        hipLaunchKernelGGL(pack_small_kernel<OP>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, src, src_is_f32,
+                           rows, cols, trans, dst, prow, pcol, items);
+        return;
+    }
     const int tiles_x = (pcol + 63) / 64, tiles_y = (prow + 63) / 64;
     const int gy = std::max(1, std::min({tiles_y, 65535, (4096 + tiles_x - 1) / tiles_x}));
+    if (items == 1) {
+        hipLaunchKernelGGL(pack_kernel<OP>, dim3((unsigned)tiles_x, (unsigned)gy), dim3(256), 0, s, src, src_is_f32, rows,
+                           cols, trans, dst, prow, pcol, ldd);
+        return;
+    }
     const int gz = std::max(1, std::min({items, 65535, 4096 / std::max(1, tiles_x * gy)}));
-    const dim3 grid((unsigned)tiles_x, (unsigned)gy, (unsigned)gz);
-    hipLaunchKernelGGL(pack_kernel<OP>, grid, dim3(256), 0, s, src, src_is_f32, rows, cols, trans, dst, prow, pcol,
-                       ldd, items);
+    hipLaunchKernelGGL(pack_items_kernel<OP>, dim3((unsigned)tiles_x, (unsigned)gy, (unsigned)gz), dim3(256), 0, s, src,
+                       src_is_f32, rows, cols, trans, dst, prow, pcol, ldd, items);
 }
 
 // Split-K.  A phase whose output tiles leave CUs idle (at most half as many
