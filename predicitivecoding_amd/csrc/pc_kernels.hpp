@@ -134,7 +134,7 @@ struct Problem {
     float prec;           // ERROR: P_{l-1}
     int slot_base;        // ERROR: first energy partial slot of this problem
     int ksplit;           // K ranges per tile (<= 1: none); the last range to finish runs the epilogue
-    int ldi;              // ERROR/UPDATE: row pitch of mlow and eself: ldo, or 0 where every row reads the first
+    int ldi;              // UPDATE: row pitch of mlow and eself: ldo, or 0 where every row reads the first
     float* part;          // split-K: fp32 partial tiles [tiles_m * tiles_n * ksplit x BM * BN]
     int* count;           // split-K: finished ranges per tile [tiles_m * tiles_n], zero between launches
 };
@@ -1777,7 +1777,7 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
             f32x4 mraw[PD][4];
             auto load_block = [&](auto Bc) PCD_INLINE {
                 constexpr int b = decltype(Bc)::value, i = b / C::FN, j = b % C::FN;
-                load_block_rows<GNT>(mraw[b % PD], P.mlow, P.ldi, row0 + wm * C::WTM + i * 32, col0 + wn * C::WTN + j * 32,
+                load_block_rows<GNT>(mraw[b % PD], P.mlow, ldo, row0 + wm * C::WTM + i * 32, col0 + wn * C::WTN + j * 32,
                                 P.M, P.N, ntld);
             };
             static_for<0, PD>([&](auto Bc) PCD_INLINE { load_block(Bc); });

@@ -765,11 +765,6 @@ int ensure_workspace(pcd_model* m, hipStream_t stream, int rows, Workspace** out
         if (l >= 1 && l <= L - 2)
             if ((st = dev_alloc_zero(w->owned, (void**)&w->E[l], (size_t)need * m->P[l] * 4))) return st;
     }
-    {
-        void* rows = nullptr;
-        if ((st = dev_alloc_zero(w->owned, &rows, front_row_bytes(m)))) return st;
-        carve_front_rows(m, w, (char*)rows);
-    }
     w->slots_cap = slots;
     if ((st = dev_alloc_zero(w->owned, (void**)&w->energy_part, (size_t)slots * need * 4))) return st;
     if ((st = dev_alloc_zero(w->owned, (void**)&w->split_part, (size_t)split_part_tiles(m) * 128 * 128 * 4)))
@@ -778,6 +773,9 @@ int ensure_workspace(pcd_model* m, hipStream_t stream, int rows, Workspace** out
     if ((st = dev_alloc_zero(w->owned, (void**)&w->act_tm, (size_t)(need / kMinTileM) * 4))) return st;
     if ((st = dev_alloc_zero(w->owned, (void**)&w->act_count, 4))) return st;
     if ((st = dev_alloc_zero(w->owned, &w->persist, kPersistBytes))) return st;
+    void* front = nullptr;
+    if ((st = dev_alloc_zero(w->owned, &front, front_row_bytes(m)))) return st;
+    carve_front_rows(m, w, (char*)front);
     HIP_TRY(hipStreamCreateWithFlags(&w->capture, hipStreamNonBlocking));
     *out = w;
     return PCD_SUCCESS;
@@ -835,7 +833,7 @@ void build_phase_sets(const pcd_model* m, const Workspace* w, int batch, Tile ti
         p.tiles_m = tm;
         p.tiles_n = (p.N + tile.n - 1) / tile.n;
         p.tiles = p.tiles_m * p.tiles_n;
-        p.ldo = p.ldi = m->P[l - 1];
+        p.ldo = m->P[l - 1];
         p.bias = m->bias[l];
         p.mlow = w->M[l - 1];
         p.eout = l - 1 >= 1 ? w->E[l - 1] : nullptr;
