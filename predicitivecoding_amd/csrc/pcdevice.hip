@@ -484,6 +484,24 @@ long error_phase_tiles(const pcd_model* m, int batch, Tile t) {
     return tiles;
 }
 
+// The most tiles of one phase at `batch` rows that a CU gets (see how
+// phase_unit deals a problem's tiles over the XCDs).
+long phase_rounds(const pcd_model* m, int batch, Tile t) {
+    const int tm = (batch + t.m - 1) / t.m, per_xcd = std::max(1, m->cus / kXcds);
+    long most = 0;
+    for (int upd = 0; upd < 2; ++upd)
+        for (int x = 0; x < kXcds; ++x) {
+            long tiles = 0;
+            for (int l = 1; l < m->L; ++l) {
+                int lo, cnt;
+                xcd_share(tm * ((m->s[l - 1 + upd] + t.n - 1) / t.n), x, lo, cnt);
+                tiles += cnt;
+            }
+            most = std::max(most, tiles);
+        }
+    return (most + per_xcd - 1) / per_xcd;
+}
+
 // The largest tile that still gives every CU at least two workgroups per
 // phase (a phase with fewer tiles leaves SIMDs idle); in fp32 fewer of 128 x 128
 // too (see there; `f32_two_per_cu`: not).  256 x 256 only for 16-bit
@@ -512,24 +530,28 @@ Tile choose_tile(const pcd_model* m, int batch, bool f32_two_per_cu = false) {
     }
     const long t128 = error_phase_tiles(m, batch, Tile{128, 128});
     if (t128 >= want) return Tile{128, 128};
-    // fp32: one 128 x 128 tile per CU is enough where the K sweeps (`mean_k` over
-    // both phases' tiles) pay its start and few of its rows are padding, since it
-    // multiplies in split bf16 (split3_tile) at 1.4 times the fp32 MFMAs' rate:
-    // 1024-wide layers at 1024 rows (256 such tiles) 6.65 ms with 64 x 64 tiles,
-    // 6.07 with 128 x 128, at 1600 rows 1.87 and 1.70 (10 steps); 3000-1500-700-300
-    // at 1024 (336) 2.42 and 2.11; but 500-wide layers at 3000 rows 0.97 and 1.02,
-    // 4096-wide ones at 260 5.22 and 5.31.  Long sweeps pay for it with idle CUs
-    // too, against three 64 x 64 tiles on a CU: 192 tiles, 4096-wide at 200 rows
-    // 4.02 and 3.64, 2048-wide at 500 2.09 and 1.98; 1024-wide at 700 1.09 and 1.16.
-    if (m->dtype == PCD_F32 && !f32_two_per_cu && 4L * batch >= 3 * (long)round_up(batch, 128)) {
-        double macs = 0, cols = 0;
+    // fp32 multiplies in split bf16 on the 128 x 128 tile (split3_tile), at 1.4
+    // times the fp32 MFMAs' rate, so fewer of them are enough, if they come out
+    // even: what counts is the most tiles a CU gets (phase_rounds).  Over 170
+    // networks and batches with half to two tiles of 128 x 128 per CU, 64 x 64
+    // -> 128 x 128 was 0.98 to 1.26 times as fast for one round against four
+    // (1.08 and more from mean K 1000 on, 1.0 at 770), 1.00 to 1.16 for two
+    // against six, 1.05 to 1.24 against seven, 1.15 to 1.30 against eight; but
+    // 0.66 to 1.05 for one against three or two (below one but for mean K 2000
+    // and more), 0.80 to 0.89 for two against four, 0.94 to 1.05 against five.
+    // Layers of unlike widths (`widest`) leave the CUs with unlike sweeps, the
+    // longest of which bounds the phase: 0.49 to 0.93 in all those cases.  A
+    // ragged settling's rounds shrink as requests leave (`f32_two_per_cu`).
+    if (m->dtype == PCD_F32 && !f32_two_per_cu) {
+        double macs = 0, cols = 0, widest = 0;
+        for (int l = 0; l < m->L; ++l) widest = std::max(widest, (double)m->s[l]);
         for (int l = 1; l < m->L; ++l) {
             macs += 2.0 * m->s[l] * m->s[l - 1];
             cols += (double)m->s[l] + m->s[l - 1];
         }
-        const double mean_k = macs / cols;
-        if (mean_k >= 640 && t128 >= m->cus) return Tile{128, 128};
-        if (mean_k >= 2048 && error_phase_tiles(m, batch, Tile{64, 64}) > want) return Tile{128, 128};
+        const double mean_k = macs / cols;   // over both phases' tiles
+        const long r64 = phase_rounds(m, batch, Tile{64, 64}), r128 = phase_rounds(m, batch, Tile{128, 128});
+        if (mean_k >= 768 && widest <= 1.5 * mean_k && r64 >= (r128 == 1 ? 4 : 3 * r128)) return Tile{128, 128};
     }
     return Tile{64, 64};
 }
@@ -2186,7 +2208,7 @@ int pcd_pc_relax_ragged(pcd_model* m, const float* x0_packed, const int* row_off
     Workspace* w = nullptr;
     if (int st = ensure_workspace(m, s, rows, &w)) return st;
     const int L = m->L;
-    const Tile tile = choose_tile(m, rows);
+    const Tile tile = choose_tile(m, rows, true);
     // Settling order: requests by decreasing step budget (stable).  As
     // requests reach their budgets the rows still running shrink towards a
     // prefix of the packing, and the row tiles past it drop out of the phases
@@ -2485,7 +2507,7 @@ int pcd_pc_classify_adaptive(pcd_model* m, const float* x0, int batch, int max_s
     RelaxSpec r;
     r.batch = rows;
     r.steps = max_steps;
-    r.tile = choose_tile(m, rows);
+    r.tile = choose_tile(m, rows, true);
     r.clamp_top = 1;
     r.row_req = d_row_req;
     r.done_at = d_done;

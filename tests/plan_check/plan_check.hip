@@ -101,6 +101,7 @@ int main(int argc, char** argv) {
         std::vector<int> sizes;
         for (int i = 3; i < argc; ++i) sizes.push_back(std::atoi(argv[i]));
         set_net(&m, sizes, std::atoi(argv[1]));
+        std::printf("tile %d\n", choose_tile(&m, std::atoi(argv[2])).m);
         bad = check(&m, std::atoi(argv[2]), true, &accepted, &sharing);
     } else {
         std::mt19937 rng((unsigned)std::atoi(argv[1]));

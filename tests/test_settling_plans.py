@@ -39,3 +39,19 @@ def test_random_plans_stay_inside_their_scratch(plan_check, seed):
     rc, out = run(plan_check, seed, 20000)
     assert rc == 0, out[-2000:]
     assert int(out.split("accepted, ")[1].split()[0]) > 10000, out   # plans with shared rows are among them
+
+
+@pytest.mark.parametrize("rows,sizes,tile", [
+    (1024, [1024] * 4 + [256], 128),     # a 128 x 128 tile on every CU, four of 64 x 64
+    (1476, [836] * 4, 64),               # 252 tiles, but 33 on some XCDs of 32 CUs
+    (1293, [1024] * 4, 64),              # 264: two rounds against four
+    (892, [1408] * 4, 128),              # 231 of 256 CUs, one round against four
+    (500, [1024] * 7, 64),               # one against three
+    (1600, [1024] * 5, 128),             # two rounds against seven
+    (892, [700] * 8, 64),                # a mean K of 700
+    (686, [107, 520, 95, 74, 84, 1724, 1281, 1494, 233], 64),   # unlike layers
+    (3000, [512] * 12, 128),             # two and more 128 x 128 tiles on every CU, whatever K
+])
+def test_fp32_tile_choice(plan_check, rows, sizes, tile):
+    _, out = run(plan_check, 0, rows, *sizes)
+    assert out.startswith(f"tile {tile}\n"), out
