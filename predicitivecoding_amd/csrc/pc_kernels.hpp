@@ -325,15 +325,15 @@ template <> __device__ __forceinline__ void mfma_chunk<f16_t>(f32x16& acc, const
 // at most what rounding that product to fp32 would cost, and 2^-27 of it in the
 // root mean square over normal operands.  Six 32x32x16 bf16 MFMAs (192 cycles)
 // replace eight 32x32x2 fp32 ones (512 cycles).  What bounds it is the power
-// limit (the matrix pipes are 63% busy at 1.73 GHz) and the splitting's VALU
-// work, 44 operations per fragment and 6 to look it over, against 24 MFMAs per
-// four fragments here;
+// limit and the splitting's VALU work (4096^3: 1.80 GHz, the matrix pipes 57%
+// busy, vector instructions issuing in 73% of the cycles), 44 operations per
+// fragment and 6 to look it over, against 24 MFMAs per four fragments here;
 // on the 64 x 64 and 32 x 32 tiles, with one block per wave, the splitting
 // outweighs what the MFMAs save (784-256-256-10 at 64 rows 267 -> 297 us,
 // 1024-wide layers at 1024 rows 6.65 -> 6.75 ms), so those keep the fp32 MFMAs,
 // as do the 256-row tiles, which have no registers left for it.  Measured, fp32
-// MFMAs -> this: 4096^3 971 -> 718 us (192 TFLOP/s), 8192^3 7.78 -> 5.7 ms, the
-// 4 x 2048 ragged batch 109 -> 78 ms.  Error against 64 bits (2-norm, normal
+// MFMAs -> this: 4096^3 974 -> 725 us (190 TFLOP/s), 1000 x 1024 x 4096 84.5 ->
+// 60.4, the 4 x 2048 ragged batch 109 -> 81.5 ms.  Error against 64 bits (2-norm, normal
 // operands): K = 64 1.4e-7 -> 5.0e-8, K = 1024 5.7e-7 -> 1.9e-7, K = 4096
 // 1.15e-6 -> 4.0e-7, K = 8192 1.6e-6 -> 5.7e-7 (one rounding of the sum per 16
 // elements of K, not one per 2).

@@ -151,7 +151,10 @@ int pool_alloc(void** out, size_t bytes, hipStream_t stream) {
         e = hipMalloc(&p, (size_t)1 << b);  // CudaAllocator.cs:43-44 fallback
         fallback = true;
     }
-    if (e != hipSuccess) return from_hip(e, "pcd_malloc_async");
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // a caller that can do without the block goes on to its launches
+        return from_hip(e, "pcd_malloc_async");
+    }
     std::lock_guard<std::mutex> g(P.mu);
     P.live[p] = {dev, b};
     if (fallback) P.synchronous[p] = true;
@@ -422,6 +425,7 @@ void free_workspace(Workspace& w) {
     w.plans.clear();
     for (void* p : w.owned) (void)hipFree(p);
     w.owned.clear();
+    w.Mr.clear();
     w.rg_tables = nullptr;
     if (w.capture) (void)hipStreamDestroy(w.capture);
     w.capture = nullptr;
@@ -754,6 +758,47 @@ size_t front_row_bytes(const pcd_model* m) {
     return carve_front_rows(m, &tmp, nullptr);
 }
 
+// One settling to enqueue: rows, steps, tile and the per-call variants.
+struct RelaxSpec {
+    int batch = 0, steps = 0;
+    Tile tile{0, 0};
+    int clamp_top = 0;              // layer L-1 holds rows staged by the caller and is never updated
+    int keep_hidden = 0;            // layers 1..L-2 start from rows staged by the caller, not from zero
+    int persistent = 0;             // the step loop as one persistent launch (see persistent_fits)
+    float* energy_out = nullptr;    // [steps x batch] per-row energies (nullable)
+    // ragged early exit (row_req null: fixed steps for every row)
+    const int* row_req = nullptr;
+    int* done_at = nullptr;
+    const int* row_offsets = nullptr;
+    int requests = 0, exit_rule = 0;
+    float exit_thr = 0.f;
+    float* prev_energy = nullptr;
+    float* last_energy = nullptr;
+};
+
+// Whether a settling computes layers the input has not reached once for the
+// whole batch (see build_front_sets).  It needs states that start the same for
+// every sample and no clamped top, a layer above the first hidden one, and
+// phases whose time follows their row tiles: on the K-shared tile and the
+// direct-weight one (and any batch of one row tile) a layer's single row takes
+// as long as its whole batch.  Elsewhere it was never slower: 0.995 to 1.42
+// times as fast over 72 networks and batches (128 to 4096 rows, fp32 and bf16).
+bool front_pays(const pcd_model* m, const RelaxSpec& r) {
+    return m->shared_rows && m->L > 2 && !r.clamp_top && !r.keep_hidden && !r.persistent && r.row_req == nullptr &&
+           r.tile.m >= 64 && !r.tile.wd && r.batch > r.tile.m;
+}
+
+// The one-row buffers of a workspace (without memory for them, settlings go
+// sample by sample; nor are they allocated while the caller records a graph).
+void ensure_front_rows(const pcd_model* m, Workspace* w, hipStream_t s) {
+    if (!w->Mr.empty()) return;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
+    void* rows = nullptr;
+    if (dev_alloc_zero(w->owned, &rows, front_row_bytes(m)) == PCD_SUCCESS) carve_front_rows(m, w, (char*)rows);
+    else (void)hipGetLastError();
+}
+
 int ensure_workspace(pcd_model* m, hipStream_t stream, int rows, Workspace** out) {
     Workspace* w = nullptr;
     for (auto& x : m->ws)
@@ -795,9 +840,13 @@ int ensure_workspace(pcd_model* m, hipStream_t stream, int rows, Workspace** out
     if ((st = dev_alloc_zero(w->owned, (void**)&w->act_tm, (size_t)(need / kMinTileM) * 4))) return st;
     if ((st = dev_alloc_zero(w->owned, (void**)&w->act_count, 4))) return st;
     if ((st = dev_alloc_zero(w->owned, &w->persist, kPersistBytes))) return st;
-    void* front = nullptr;
-    if ((st = dev_alloc_zero(w->owned, &front, front_row_bytes(m)))) return st;
-    carve_front_rows(m, w, (char*)front);
+    // Here for a workspace whose largest settling shares rows; one whose settlings
+    // run on the small tiles does without (a settling that an option gives a
+    // larger tile allocates them itself).
+    RelaxSpec largest;
+    largest.batch = need;
+    largest.tile = choose_tile(m, need);
+    if (front_pays(m, largest)) ensure_front_rows(m, w, stream);
     HIP_TRY(hipStreamCreateWithFlags(&w->capture, hipStreamNonBlocking));
     *out = w;
     return PCD_SUCCESS;
@@ -808,24 +857,6 @@ int ensure_workspace(pcd_model* m, hipStream_t stream, int rows, Workspace** out
 const void* state_operand(const pcd_model* m, const Workspace* w, int l) {
     return m->dtype == PCD_F32 ? (const void*)w->M[l] : w->S[l];
 }
-
-// One settling to enqueue: rows, steps, tile and the per-call variants.
-struct RelaxSpec {
-    int batch = 0, steps = 0;
-    Tile tile{0, 0};
-    int clamp_top = 0;              // layer L-1 holds rows staged by the caller and is never updated
-    int keep_hidden = 0;            // layers 1..L-2 start from rows staged by the caller, not from zero
-    int persistent = 0;             // the step loop as one persistent launch (see persistent_fits)
-    float* energy_out = nullptr;    // [steps x batch] per-row energies (nullable)
-    // ragged early exit (row_req null: fixed steps for every row)
-    const int* row_req = nullptr;
-    int* done_at = nullptr;
-    const int* row_offsets = nullptr;
-    int requests = 0, exit_rule = 0;
-    float exit_thr = 0.f;
-    float* prev_energy = nullptr;
-    float* last_energy = nullptr;
-};
 
 // Problem sets of the two phases for a batch; problems beyond kMaxProblems
 // spill into further sets (still one phase: the problems are independent).
@@ -895,16 +926,9 @@ void build_phase_sets(const pcd_model* m, const Workspace* w, int batch, Tile ti
     *nslots = slot;
 }
 
-// Whether a settling computes layers the input has not reached once for the
-// whole batch (see build_front_sets).  It needs states that start the same for
-// every sample and no clamped top, a layer above the first hidden one, and
-// phases whose time follows their row tiles: on the K-shared tile and the
-// direct-weight one (and any batch of one row tile) a layer's single row takes
-// as long as its whole batch.  Elsewhere it was never slower: 0.995 to 1.42
-// times as fast over 72 networks and batches (128 to 4096 rows, fp32 and bf16).
+// Whether a settling does so: where it pays and its workspace has the one-row buffers.
 bool use_front(const pcd_model* m, const Workspace* w, const RelaxSpec& r) {
-    return m->shared_rows && !w->Mr.empty() && m->L > 2 && !r.clamp_top && !r.keep_hidden && !r.persistent && r.row_req == nullptr &&
-           r.tile.m >= 64 && !r.tile.wd && r.batch > r.tile.m;
+    return !w->Mr.empty() && front_pays(m, r);
 }
 
 // Problem sets of step t < L - 1 of a settling from equal free states.  The
@@ -1314,6 +1338,7 @@ int run_relax(pcd_model* m, Workspace* w, int batch, int steps, int clamp_top, i
     r.tile = choose_tile(m, batch);
     r.clamp_top = clamp_top;
     r.keep_hidden = keep_hidden;
+    if (front_pays(m, r)) ensure_front_rows(m, w, s);
     *energy = nullptr;
     if (!want_energy || caller_energy) {
         r.energy_out = want_energy ? caller_energy : nullptr;
@@ -2071,8 +2096,9 @@ int scratch_device(int device, ScratchDevice** out) {
 // Lays out the workspace of a `batch`-row settling with `tile` from `base`:
 // the buffers ensure_workspace allocates (energy slots for this tile only),
 // then split-K scratch for exactly the partial tiles this call's phases use
-// (the split plan itself is the allocating path's, so the kernels and their
-// results are the same).  Returns the bytes the layout spans.
+// (the split plan itself is the allocating path's, so with its tile and
+// `front_rows` as its option says the kernels and their results are the same).
+// Returns the bytes the layout spans.
 size_t carve_workspace(const pcd_model* m, char* base, int batch, Tile tile, bool front_rows, Workspace& w) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
