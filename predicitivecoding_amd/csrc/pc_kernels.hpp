@@ -1218,32 +1218,39 @@ __device__ __forceinline__ void phase_unit(KProblem* kprobs, const int nprob, co
     // the B source by KE rows.  A transposed A (AKM) fills the A region (KE
     // rows of BM elements) the same way.
     const char* src[C::QPW];
-#pragma unroll
-    for (int i = 0; i < C::QPW; ++i) {
-        const int q = wave_u * C::QPW + i;
-        const int R = q * C::ROWS_PER_LOAD + lane / C::UNITS;
-        const int unit = swz<C::RB>(R, lane % C::UNITS);
-        // A product's last tiles repeat its last row, or the last unit of a K
-        // row, where they reach past it (those results are not stored), so the
-        // caller's operands need no whole tiles.
+    // In a product's last tiles, which reach past it, a row or column repeats the
+    // last one, and a unit of a K row the last unit (those results are not
+    // stored), so the caller's operands need no whole tiles.  (Elsewhere the
+    // addresses are one row's and constant steps from it.)
+    constexpr bool edges = EPI >= EPI_PLAIN;
+    auto set_sources = [&](auto Clamp) PCD_INLINE {
+        constexpr bool clamp = decltype(Clamp)::value;
         constexpr int UE = 16 / OPB;   // elements of a unit
-        if (BKN && R >= BM) {
-            const int ob = (q * C::ROWS_PER_LOAD - BM) * C::RB + lane * 16;
-            const int kr = kn_row<BN, OPB>(ob / (BN * OPB));
-            const int at = kn_unit<BN, OPB>(kr, (ob % (BN * OPB)) / 16) * UE;
-            src[i] = Bg + (size_t)kr * ldb_b + (ptrdiff_t)(min(col0 + at, P.N - UE) - col0) * OPB;
-        } else if (AKM && R < BM) {
-            const int ob = q * C::ROWS_PER_LOAD * C::RB + lane * 16;
-            const int kr = kn_row<BM, OPB>(ob / (BM * OPB));
-            const int at = kn_unit<BM, OPB>(kr, (ob % (BM * OPB)) / 16) * UE;
-            src[i] = Ag + (size_t)kr * lda_b + (ptrdiff_t)(min(row0 + at, P.M - UE) - row0) * OPB;
-        } else if (EPI >= EPI_PLAIN) {
-            src[i] = (R < BM ? Ag + (size_t)(min(row0 + R, P.M - 1) - row0) * lda_b
-                             : Bg + (size_t)(min(col0 + R - BM, P.N - 1) - col0) * ldb_b) + unit * 16;
-        } else {
-            src[i] = R < BM ? Ag + (size_t)R * lda_b + unit * 16 : Bg + (size_t)(R - BM) * ldb_b + unit * 16;
+#pragma unroll
+        for (int i = 0; i < C::QPW; ++i) {
+            const int q = wave_u * C::QPW + i;
+            const int R = q * C::ROWS_PER_LOAD + lane / C::UNITS;
+            const int unit = swz<C::RB>(R, lane % C::UNITS);
+            if (BKN && R >= BM) {
+                const int ob = (q * C::ROWS_PER_LOAD - BM) * C::RB + lane * 16;
+                const int kr = kn_row<BN, OPB>(ob / (BN * OPB));
+                const int at = kn_unit<BN, OPB>(kr, (ob % (BN * OPB)) / 16) * UE;
+                src[i] = Bg + (size_t)kr * ldb_b + (ptrdiff_t)(clamp ? min(col0 + at, P.N - UE) - col0 : at) * OPB;
+            } else if (AKM && R < BM) {
+                const int ob = q * C::ROWS_PER_LOAD * C::RB + lane * 16;
+                const int kr = kn_row<BM, OPB>(ob / (BM * OPB));
+                const int at = kn_unit<BM, OPB>(kr, (ob % (BM * OPB)) / 16) * UE;
+                src[i] = Ag + (size_t)kr * lda_b + (ptrdiff_t)(clamp ? min(row0 + at, P.M - UE) - row0 : at) * OPB;
+            } else if (clamp) {
+                src[i] = (R < BM ? Ag + (size_t)(min(row0 + R, P.M - 1) - row0) * lda_b
+                                 : Bg + (size_t)(min(col0 + R - BM, P.N - 1) - col0) * ldb_b) + unit * 16;
+            } else {
+                src[i] = R < BM ? Ag + (size_t)R * lda_b + unit * 16 : Bg + (size_t)(R - BM) * ldb_b + unit * 16;
+            }
         }
-    }
+    };
+    if (edges && (row0 + BM > P.M || col0 + BN > P.N)) set_sources(std::true_type{});
+    else set_sources(std::false_type{});
     const size_t bstep = BKN ? (size_t)KE * ldb_b : (size_t)C::RB;   // source bytes per stage of B loads
     const size_t astep = AKM ? (size_t)KE * lda_b : (size_t)C::RB;   // ... and of A loads
     auto issue_stage = [&](int kt) PCD_INLINE {

@@ -1595,8 +1595,13 @@ int pcd_event_elapsed_ms(float* ms, void* start, void* end) {
 // With fewer 128 x 128 tiles than CUs that tile is still the faster one where
 // some CU would get a third 64 x 64 tile and K is long enough to pay its start
 // (64 x 64 -> 128 x 128: 1300 x 3000 x 2000 bf16 51.6 -> 45.9 us, fp32 171 -> 146;
-// 1700 x 600 x 1500 25.2 -> 24.8 and 49.8 -> 47.4; 1600 x 512 x 1600 12.2 -> 13.1
-// and 32 -> 33 to 36), and in fp32, where it multiplies at 1.4 times the other
+// 1700 x 600 x 1500 fp32 49.8 -> 47.4; 1600 x 512 x 1600 12.2 -> 13.1 and 32 -> 33
+// to 36; in 16 bits from K 704 on, 3072 x 640 x 832 12.4 -> 12.8, 1536 x 704 x
+// 2560 15.0 -> 12.7) -- but not in 16 bits for an operand in K rows that the 64 x
+// 64 tile reads in place and the 128 x 128 tile would pack or, with K below 1024,
+// reads too slowly (`k_rows`: 4608 x 1280 x 768 22.5 -> 25.5, 3200 x 1152 x 768, A
+// transposed, 18.5 -> 23.3, 2240 x 896 x 1344 15.8 -> 16.4; 1152 x 1344 x 3520
+// 23.9 -> 21.2) -- and in fp32, where it multiplies at 1.4 times the other
 // tiles' rate, wherever K ranges of 1024 and more spread it over the CUs (1024 x
 // 4096 x 1024 90 -> 66 us, 256 x 8192 x 4096 181 -> 117, 640 x 8192 x 640 95 ->
 // 67; ranges of 400 lose: 300 x 2048 x 2048 33 -> 36).  Error against 64 bits
@@ -1609,13 +1614,13 @@ int pcd_event_elapsed_ms(float* ms, void* start, void* end) {
 // stored non-temporally: a caller reads them long after the L2 has turned over.
 constexpr size_t kGemmNtBytes = (size_t)64 << 20;
 
-static Tile choose_gemm_tile(int dtype, int m, int k, int n, int cus, int batch = 1) {
+static Tile choose_gemm_tile(int dtype, int m, int k, int n, int cus, int batch, bool k_rows) {
     auto tiles = [&](int t) { return (long)batch * ((m + t - 1) / t) * ((n + t - 1) / t); };
     auto fits = [&](int t) { return t <= (int)round_up(m, 64) && t <= (int)round_up(n, 64); };
     if (dtype != PCD_F32 && fits(256) && tiles(256) >= cus) return Tile{256, 256};
     if (fits(128) && tiles(128) >= cus) return Tile{128, 128};
     if (fits(128) && 4L * m * n * batch >= 3L * tiles(128) * 128 * 128) {   // at most a quarter of it padding
-        if (k >= 640 && tiles(64) > 2L * cus) return Tile{128, 128};
+        if (k >= (dtype == PCD_F32 ? 640 : 704) && !k_rows && tiles(64) > 2L * cus) return Tile{128, 128};
         const long split = std::min<long>(kMaxSplit, cus / tiles(128));
         if (dtype == PCD_F32 && batch == 1 && tiles(128) * split * 4 >= 3L * cus && k / split >= 1024)
             return Tile{128, 128};
@@ -1647,25 +1652,36 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     int dev = 0, cus = 256;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const Tile tile = choose_gemm_tile(dtype, m, k, n, cus, batch);
     const int ob = op_bytes(dtype), unit = 16 / ob;
-    const int kp = (int)round_up(k, stage_k(dtype, tile));
     const uintptr_t c0 = (uintptr_t)dC, c1 = c0 + (size_t)batch * m * n * 4;
     auto in_place = [&](const void* p, size_t item) {
         const uintptr_t p0 = (uintptr_t)p, p1 = p0 + (size_t)batch * item * ob;
         return p0 % 16 == 0 && (batch == 1 || item * ob % 16 == 0) && (p1 <= c0 || c1 <= p0);
     };
+    // Operands in K rows that can be read in place if K is whole stages.
+    const bool rows_a = trans_a && m % unit == 0 && in_place(dA, (size_t)m * k);
+    const bool rows_b = !trans_b && n % unit == 0 && in_place(dB, (size_t)k * n);
+    const bool k_rows = ob == 2 && k % stage_k(dtype, Tile{64, 64}) == 0 &&
+                        ((rows_a && (k < 1024 || (size_t)m * 4 <= (size_t)n)) ||
+                         (rows_b && (k < 1024 || (size_t)n * 4 <= (size_t)m)));
+    const Tile tile = choose_gemm_tile(dtype, m, k, n, cus, batch, k_rows);
+    const int kp = (int)round_up(k, stage_k(dtype, tile));
     // Except that the transposing reads cost the 16-bit 128 x 128 tile about a
     // fifth of its time, more than packing an operand a quarter the other's size
     // or smaller takes (512 x 8192 x 8192 bf16, A transposed: 0.089 ms in place,
-    // 0.081 packed; the other tiles lose 2-5% and read in place).
-    const bool small_a = ob == 2 && tile.m == 128 && (size_t)m * 4 <= (size_t)n;
-    const bool small_b = ob == 2 && tile.m == 128 && (size_t)n * 4 <= (size_t)m;
+    // 0.081 packed; the other tiles lose 2-5% and read in place); and the reads of
+    // single elements the fp32 32 x 32 tile a twentieth to a fifth, more than
+    // packing a much smaller operand beside a K-contiguous one once the product is
+    // long (3104 x 6976 x 36 49.7 us in place, 40.1 packed; 5032 x 2624 x 132 62.3,
+    // 57.2; 1324 x 3200 x 152 25.3, 25.2; but 1556 x 1088 x 300 17.8, 20.5).
+    const bool mid = ob == 2 && tile.m == 128;
+    const bool long32 = tile.m == 32 && k >= 2560 && (double)m * n * k >= 6e8;
+    const bool small_a = (mid && (size_t)m * 4 <= (size_t)n) || (long32 && trans_b && (size_t)m * 5 <= (size_t)n * 2);
+    const bool small_b = (mid && (size_t)n * 4 <= (size_t)m) || (long32 && !trans_a && (size_t)n * 5 <= (size_t)m * 2);
     const bool whole_k = k == kp, kn = whole_k && kn_tile(ob, tile.m, tile.n, false);
     const bool direct_a = whole_k && !trans_a && k % unit == 0 && in_place(dA, (size_t)m * k);
     const bool direct_b = whole_k && trans_b && k % unit == 0 && in_place(dB, (size_t)k * n);
-    const bool mk_a = kn && trans_a && !small_a && m % unit == 0 && in_place(dA, (size_t)m * k);
-    const bool kn_b = kn && !trans_b && !small_b && n % unit == 0 && in_place(dB, (size_t)k * n);
+    const bool mk_a = kn && rows_a && !small_a, kn_b = kn && rows_b && !small_b;
     void *pa = nullptr, *pb = nullptr, *part = nullptr;
     auto pack = [&](const void* src, int rows, int trans, void* dst) -> int {
         const int f32 = dtype == PCD_F32;

@@ -60,3 +60,34 @@ def test_settlings_near_the_tile_rules(width, rows):
     for a, c in zip(*out):   # fp32 sums of up to 2048 products in two orders, six steps of them
         assert ((a - c).norm() / c.norm()).item() <= 6 * 2.0 ** -24 * np.sqrt(2048)
     model.close()
+
+
+@pytest.mark.parametrize("m,k,n", [(3072, 1024, 768), (2048, 960, 1408), (1792, 1024, 1408), (1536, 704, 2560),
+                                   (1536, 640, 2560), (4608, 1280, 768)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_16_bit_products_near_the_rules_for_k_rows(dtype, m, k, n, ta, tb):
+    """Operands in K rows small and large, K on both sides of 1024 and 704; every one packed as well (one element off
+    its alignment), whichever tile that takes."""
+    check_layouts(dtype, m, k, n, ta, tb)
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb", [(1500, 2560, 160, 0, 0), (1500, 2496, 160, 0, 0), (400, 2560, 1000, 1, 1),
+                                         (404, 2560, 1000, 1, 1), (1460, 2560, 160, 0, 0), (1500, 2560, 160, 1, 0)])
+def test_fp32_products_near_the_rule_that_packs_a_small_operand(m, k, n, ta, tb):
+    """K on both sides of 2560, 6e8 multiply-adds and less, an operand two fifths of the other and a bit more."""
+    check_layouts("f32", m, k, n, ta, tb)
+
+
+def check_layouts(dtype, m, k, n, ta, tb):
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    A = torch.randn((k, m) if ta else (m, k), device="cuda", generator=g).to(TORCH[dtype])
+    B = torch.randn((n, k) if tb else (k, n), device="cuda", generator=g).to(TORCH[dtype])
+    a, b = (A.double().T if ta else A.double()), (B.double().T if tb else B.double())
+    off = [torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:] for t in (A, B)]
+    for x, y in ((A, B), off):
+        C = torch.full((m, n), float("nan"), device="cuda")
+        call(f"pcd_gemm_{dtype}", x.data_ptr(), y.data_ptr(), C.data_ptr(), m, k, n, ta, tb, 0.0, None)
+        torch.cuda.synchronize()
+        # a rounding of 2^-24 of the running sum per two elements of K, independent ones adding in the square
+        assert ((C.double() - a @ b).norm() / (a @ b).norm()).item() <= 2.0 ** -24 * np.sqrt(k / 2 + 2)
