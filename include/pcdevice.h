@@ -146,10 +146,11 @@ int pcd_event_elapsed_ms(float* ms, void* start, void* end);
  * CudaGemmProvider.MatMulDeviceEx (Gemm/CudaGemmProvider.cs:82-98): op(A) is
  * A [m,k] or, with trans_a, the transpose of a physical [k,m] A (same for B).
  * With trans_a = trans_b = 0 and beta = 0 this is MatMulDevice (:62-72).
- * Operands are read where they lie when aligned and whole-tile shaped
- * (16-bit operands in either layout: a row-major B or a transposed A is
- * transposed in LDS); others, and one that C overwrites,
- * are packed into scratch from the library's pool. */
+ * An operand of any type and layout is read where it lies when its rows and
+ * its address are 16-byte aligned and k is a whole number of the tile's stages
+ * (a multiple of 64 always is; no whole tiles of rows or columns needed); any
+ * other, a small one beside a large one in some 16-bit products, and one that
+ * C overwrites, is packed into scratch from the library's pool. */
 int pcd_gemm_f32(const float* dA, const float* dB, float* dC, int m, int k, int n,
                  int trans_a, int trans_b, float beta, void* stream);
 /* bf16 operands (raw bf16 bit patterns), fp32 accumulation and fp32 C:
@@ -208,13 +209,17 @@ int pcd_pc_relax(pcd_model* model, const float* x0, int batch, int steps,
 
 /* No counterpart in the reference: pcd_pc_relax for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc).  Same arguments, kernels and results as
- * pcd_pc_relax, but the call allocates nothing: its scratch (states, deltas,
+ * harnesses that forbid hipMalloc).  Same arguments, kernels and results (to
+ * the bit, but near the array's end, below) as pcd_pc_relax, but the call
+ * allocates nothing: its scratch (states, deltas,
  * energy partials, split-K partial tiles) lives in a library-owned device
  * array of 64 MiB per device, which each device holds until the process ends,
  * and the step loop runs as plain kernel launches (no cached graph).  A call
  * whose batch needs more scratch than that fails with PCD_INVALID_VALUE
- * before launching anything (pcd_last_error names the size).  Every call on a
+ * before launching anything (pcd_last_error names the size); one that fits
+ * only without the rows that option shared_rows keeps, or with a smaller fp32
+ * tile, runs without them, and its results then agree with pcd_pc_relax's to
+ * rounding (16-bit models, and fp32 where the tile differs).  Every call on a
  * device shares that device's array: the library runs such calls one after
  * another, whatever their streams, threads or models (each call's stream waits
  * on an event the previous call recorded, set up with the array on the first
