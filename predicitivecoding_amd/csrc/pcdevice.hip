@@ -1665,7 +1665,15 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
                         ((rows_a && (k < 1024 || (size_t)m * 4 <= (size_t)n)) ||
                          (rows_b && (k < 1024 || (size_t)n * 4 <= (size_t)m)));
     const Tile tile = choose_gemm_tile(dtype, m, k, n, cus, batch, k_rows);
+    // kp: the sweep's K, whole stages.  kl: the pitch of a packed operand's rows,
+    // whole 128-byte lines for the long sweeps of the 16-bit tiles of 64-byte
+    // stages, whose rows would else begin within a line (2944 x 2130 x 2048 64.2
+    // us at the pitch 2144, 61.2 at 2176; 2765 x 3277 x 1455 85.7 and 78.6; 19
+    // products of K from 1200 0.98 to 1.11 times as fast, 1.03 in the mean).  K
+    // from 400 to 1200 gains half a percent; below, what the packing writes more
+    // costs up to 6%, and the fp32 tile's sweep hides it (0.97 to 1.01).
     const int kp = (int)round_up(k, stage_k(dtype, tile));
+    const int kl = ob == 2 && tile.m >= 128 && k >= 512 ? (int)round_up(kp, 64) : kp;
     // Except that the transposing reads cost the 16-bit 128 x 128 tile about a
     // fifth of its time, more than packing an operand a quarter the other's size
     // or smaller takes (512 x 8192 x 8192 bf16, A transposed: 0.089 ms in place,
@@ -1686,25 +1694,25 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     auto pack = [&](const void* src, int rows, int trans, void* dst) -> int {
         const int f32 = dtype == PCD_F32;
         switch (dtype) {
-        case PCD_F32: pack_op<float>(s, src, f32, rows, k, trans, dst, rows, kp, kp, batch); break;
-        case PCD_BF16: pack_op<bf16_t>(s, src, f32, rows, k, trans, dst, rows, kp, kp, batch); break;
-        default: pack_op<f16_t>(s, src, f32, rows, k, trans, dst, rows, kp, kp, batch); break;
+        case PCD_F32: pack_op<float>(s, src, f32, rows, k, trans, dst, rows, kl, kl, batch); break;
+        case PCD_BF16: pack_op<bf16_t>(s, src, f32, rows, k, trans, dst, rows, kl, kl, batch); break;
+        default: pack_op<f16_t>(s, src, f32, rows, k, trans, dst, rows, kl, kl, batch); break;
         }
         return from_hip(hipGetLastError(), "pack_kernel launch");
     };
     int st = PCD_SUCCESS;
     if (!direct_a && !mk_a)
-        if (!(st = pool_alloc(&pa, (size_t)batch * m * kp * ob, s))) st = pack(dA, m, trans_a, pa);
+        if (!(st = pool_alloc(&pa, (size_t)batch * m * kl * ob, s))) st = pack(dA, m, trans_a, pa);
     if (!st && !direct_b && !kn_b)
-        if (!(st = pool_alloc(&pb, (size_t)batch * n * kp * ob, s))) st = pack(dB, n, !trans_b, pb);
+        if (!(st = pool_alloc(&pb, (size_t)batch * n * kl * ob, s))) st = pack(dB, n, !trans_b, pb);
     std::vector<ProblemSet> sets(1);
     std::memset(&sets[0], 0, sizeof(ProblemSet));
     sets[0].n = 1;
     Problem& p = sets[0].p[0];
     p.A = pa ? pa : dA;
-    p.lda = mk_a ? m : kp;   // the row pitch of a transposed A, else of the K-contiguous rows
+    p.lda = mk_a ? m : pa ? kl : k;   // the row pitch of a transposed A, else of the K-contiguous rows
     p.B = pb ? pb : dB;
-    p.ldb = kn_b ? n : kp;   // the row pitch of row-major B, else of the K-contiguous copy
+    p.ldb = kn_b ? n : pb ? kl : k;   // the row pitch of row-major B, else of the K-contiguous rows
     p.M = m;
     p.N = n;
     p.K = kp;
@@ -1752,8 +1760,8 @@ static int gemm_common(int dtype, const void* dA, const void* dB, float* dC, int
     a.beta = beta;
     a.k_stagger = dtype == PCD_F32 ? 0 : auto_k_stagger(kp / stage_k(dtype, tile));
     a.nt_store = (size_t)batch * m * n * 4 >= kGemmNtBytes;
-    p.item_a = (size_t)m * kp * ob;
-    p.item_b = (size_t)n * kp * ob;
+    p.item_a = (size_t)m * (pa ? kl : k) * ob;
+    p.item_b = (size_t)n * (pb ? kl : k) * ob;
     p.item_c = (size_t)m * n;
     const int epi = mk_a ? (kn_b ? EPI_PLAIN_MKKN : EPI_PLAIN_MK) : (kn_b ? EPI_PLAIN_KN : EPI_PLAIN);
     // Launches of at most 2^22 work units (one, but for batches of millions):
